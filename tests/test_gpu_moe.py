@@ -141,6 +141,53 @@ def test_moe_route(gpu):
     np.testing.assert_allclose(sg.cpu().numpy(), ref_sg, rtol=1e-5)
 
 
+@pytest.mark.parametrize("P", [1, 3, 257, 1027])
+def test_moe_route_batches(gpu, P):
+    """Every positions-a-workgroup form (1, 4, 8) with a ragged last workgroup: logits in float64 decide
+    the ids where the 8th and 9th are apart by more than fp32 sums of 2048 terms can move (1e-4)."""
+    print(f"[case] moe route P={P}", flush=True)
+    rng = np.random.default_rng(1200 + P)
+    wrt = (rng.standard_normal((moe.E, moe.HID)) * 0.02).astype(np.float32)
+    wsh = (rng.standard_normal(moe.HID) * 0.02).astype(np.float32)
+    h = rng.standard_normal((P, moe.HID)).astype(np.float32)
+    eids = torch.full((P + 1, 8), -1, dtype=torch.int16, device=gpu)
+    gates = torch.full((P + 1, 8), -1.0, device=gpu)
+    sg = torch.full((P + 1,), -1.0, device=gpu)
+    ops.moe_route(torch.from_numpy(wrt).to(gpu), torch.from_numpy(wsh).to(gpu), torch.from_numpy(h).to(gpu),
+                  eids, gates, sg)
+    torch.cuda.synchronize()
+    assert (eids[P] == -1).all() and (gates[P] == -1).all() and sg[P] == -1   # nothing past the last position
+    lg = h.astype(np.float64) @ wrt.astype(np.float64).T
+    order = np.argsort(-lg, axis=1, kind="stable")[:, :9]
+    top = np.take_along_axis(lg, order, 1)
+    clear = np.min(-np.diff(top, axis=1), axis=1) > 1e-4
+    assert clear.sum() >= P // 2
+    assert np.array_equal(eids[:P].cpu().numpy()[clear], order[clear, :8].astype(np.int16))
+    ex = np.exp(top[:, :8] - top[:, :1])
+    np.testing.assert_allclose(gates[:P].cpu().numpy()[clear], (ex / ex.sum(1, keepdims=True))[clear], rtol=1e-4)
+    ref = 1.0 / (1.0 + np.exp(-(h.astype(np.float64) @ wsh.astype(np.float64))))
+    np.testing.assert_allclose(sg[:P].cpu().numpy(), ref, rtol=1e-5)
+
+
+def test_moe_topk_extremes(gpu):
+    """Ties over every lane, infinities and the mask's own value: the oracle's ids (lower id first)."""
+    print("[case] moe topk extremes", flush=True)
+    lg = np.zeros((5, moe.E), np.float32)                     # all equal: ids 0..7
+    lg[1] = -np.arange(moe.E)                                 # one lane holds the first four
+    lg[2] = np.arange(moe.E)[::-1] // 3                       # ties of three across lanes
+    lg[3, ::2], lg[3, 1::2] = -0.0, 0.0                       # zeros of both signs are equal
+    lg[4] = -3.0e38
+    lg[4, 255] = 3.0e38
+    eids = torch.empty(5, 8, dtype=torch.int16, device=gpu)
+    gates = torch.empty(5, 8, device=gpu)
+    ops.moe_topk(torch.from_numpy(lg).to(gpu), eids, gates)
+    torch.cuda.synchronize()
+    ref_e, ref_g = moe.topk_ref(lg)
+    assert np.array_equal(eids.cpu().numpy().view(np.uint16), ref_e)
+    np.testing.assert_allclose(gates.cpu().numpy(), ref_g, rtol=2e-6, atol=1e-7)
+
+
+
 @pytest.mark.parametrize("P", [11, 2048])
 def test_moe_sort(gpu, P):
     print(f"[case] moe sort P={P}", flush=True)

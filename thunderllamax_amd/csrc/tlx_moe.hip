@@ -30,145 +30,160 @@ constexpr int kE = 256, kTopK = 8, kHid = 2048, kFf = 512;
 constexpr int kGateBytes = kFf * 1088;     // GATE_B4
 
 // ------------------------------------------------------------------ router
-// 8 masked-argmax passes over one position's 256 logits held 4 per lane (lane l: experts
-// l, l+64, l+128, l+192), wave-wide: larger value wins, equal values go to the lower id.
-__device__ __forceinline__ void topk8_wave(float v[4], int lane, uint16_t* eids, float* gates) {
-  float m = -3.402823466e38f, ex[kTopK], s8 = 0.f;
-  int ids[kTopK];
+// A wave's reductions by DPP: quad swaps, half-row and row mirrors leave each 16-lane row its result
+// in every lane; two row broadcasts carry rows 0-2 into row 3, so lane 63 holds the wave's.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_f(float v) {   // lanes outside ROWS keep v
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ float lane63(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+__device__ __forceinline__ float wave_max(float v) {   // (fmaxf: NaN only if every lane's is)
+  v = fmaxf(v, dpp_f<0xB1, 0xF>(v));
+  v = fmaxf(v, dpp_f<0x4E, 0xF>(v));
+  v = fmaxf(v, dpp_f<0x141, 0xF>(v));
+  v = fmaxf(v, dpp_f<0x140, 0xF>(v));
+  v = fmaxf(v, dpp_f<0x142, 0xA>(v));   // row_bcast:15 into rows 1 and 3
+  v = fmaxf(v, dpp_f<0x143, 0xC>(v));   // row_bcast:31 into rows 2 and 3
+  return lane63(v);
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  v += dpp_f<0xB1, 0xF>(v);
+  v += dpp_f<0x4E, 0xF>(v);
+  v += dpp_f<0x141, 0xF>(v);
+  v += dpp_f<0x140, 0xF>(v);
+  const float r15 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));
+  v += r15;   // (0 in rows 0 and 2)
+  const float r31 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));
+  v += r31;
+  return lane63(v);
+}
+
+// Top-8 of one position by a wave, lane l holding experts 4 l .. 4 l + 3 in v: 8 passes, each the
+// wave's largest value and, among the experts that equal it, the lowest id (the first lane of a
+// ballot, then its first element: scalar work), which is masked for the passes after.  A pass is 9
+// dependent vector steps and four compares; exchanging (value, id) pairs lane by lane took 15 + 4
+// compare-and-select pairs a pass on a 16-lane row.  Softmax over the 8, summed in pass order.  A
+// NaN is never chosen before a number (a position of NaNs takes ids 0, 1, .. and NaN gates).
+__device__ __forceinline__ void topk8_wave(float4 in, int lane, uint16_t* eids, float* gates) {
+  float v[4] = {in.x, in.y, in.z, in.w};
+  int id = 0;
+  float val = 0.f, first = 0.f;
 #pragma unroll
   for (int r = 0; r < kTopK; ++r) {
-    float bv = v[0];
-    int bi = lane;
+    const float m = wave_max(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+    if (r == 0) first = m;
+    uint64_t eq[4];
 #pragma unroll
-    for (int j = 1; j < 4; ++j)
-      if (v[j] > bv) { bv = v[j]; bi = lane + 64 * j; }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
-    if (r == 0) m = bv;
-    ids[r] = bi;
-    ex[r] = expf(bv - m);
-    s8 += ex[r];
+    for (int j = 0; j < 4; ++j) eq[j] = __ballot(v[j] == m);
+    const uint64_t any = eq[0] | eq[1] | eq[2] | eq[3];
+    const int at = any ? __builtin_ctzll(any) : 0;
+    const int j0 = (eq[0] >> at) & 1 ? 0 : (eq[1] >> at) & 1 ? 1 : (eq[2] >> at) & 1 ? 2 : 3;
+    const int best = any ? 4 * at + j0 : r;
+    if (lane == r) { id = best; val = m; }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (bi == lane + 64 * j) v[j] = -3.402823466e38f;
+      if (4 * lane + j == best) v[j] = -3.402823466e38f;
   }
-  if (lane < kTopK) {
-    int id = ids[0];
-    float e = ex[0];
+  const float e = expf(val - first);
+  float s8 = 0.f;
 #pragma unroll
-    for (int r = 1; r < kTopK; ++r)
-      if (lane == r) { id = ids[r]; e = ex[r]; }
+  for (int r = 0; r < kTopK; ++r) s8 += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), r));
+  if (lane < kTopK) {
     eids[lane] = (uint16_t)id;
     gates[lane] = e / s8;
   }
 }
 
-// The same 8 passes with a position per 16-lane row (lane l: experts 16 l .. 16 l + 15): the row's
-// argmax is 4 DPP exchange steps inside the row (quad swaps, half-row and row mirrors) instead of
-// 6 cross-lane shuffles over the wave, which go through the LDS crossbar and serialize 96 round
-// trips per position.  Same comparisons, same order of the softmax sums: the same results.
-template <int CTRL>
-__device__ __forceinline__ void argmax_dpp_step(float& bv, int& bi) {
-  const float ov = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, bv), CTRL, 0xF, 0xF, true));
-  const int oi = __builtin_amdgcn_update_dpp(0, bi, CTRL, 0xF, 0xF, true);
-  if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-}
-
-__device__ __forceinline__ void topk8_row16(const float4 (&in)[4], int l, uint16_t* eids, float* gates) {
-  float v[16];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) { v[4 * q] = in[q].x; v[4 * q + 1] = in[q].y; v[4 * q + 2] = in[q].z; v[4 * q + 3] = in[q].w; }
-  float m = -3.402823466e38f, ex[kTopK], s8 = 0.f;
-  int ids[kTopK];
-#pragma unroll
-  for (int r = 0; r < kTopK; ++r) {
-    float bv = v[0];
-    int bi = 16 * l;
-#pragma unroll
-    for (int j = 1; j < 16; ++j)
-      if (v[j] > bv) { bv = v[j]; bi = 16 * l + j; }
-    argmax_dpp_step<0xB1>(bv, bi);    // quad_perm [1, 0, 3, 2]
-    argmax_dpp_step<0x4E>(bv, bi);    // quad_perm [2, 3, 0, 1]
-    argmax_dpp_step<0x141>(bv, bi);   // row_half_mirror: quad q with quad 1 - q of each half
-    argmax_dpp_step<0x140>(bv, bi);   // row_mirror: half with half
-    if (r == 0) m = bv;
-    ids[r] = bi;
-    ex[r] = expf(bv - m);
-    s8 += ex[r];
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-      if (bi == 16 * l + j) v[j] = -3.402823466e38f;
-  }
-  if (l < kTopK) {
-    int id = ids[0];
-    float e = ex[0];
-#pragma unroll
-    for (int r = 1; r < kTopK; ++r)
-      if (l == r) { id = ids[r]; e = ex[r]; }
-    eids[l] = (uint16_t)id;
-    gates[l] = e / s8;
-  }
-}
-
-// a position per 16-lane row, 16 positions per 256-thread workgroup
+// a position per wave, 4 per workgroup
 __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__ logits, uint16_t* __restrict__ eids,
                                                        float* __restrict__ gates, int P) {
-  const int p = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;
-  if (p >= P) return;   // whole 16-lane rows: the exchanges stay inside a row
-  float4 in[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) in[q] = reinterpret_cast<const float4*>(logits + (size_t)p * kE + 16 * l)[q];
-  topk8_row16(in, l, eids + (size_t)p * kTopK, gates + (size_t)p * kTopK);
+  const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (p >= P) return;
+  topk8_wave(reinterpret_cast<const float4*>(logits + (size_t)p * kE)[lane], lane, eids + (size_t)p * kTopK,
+             gates + (size_t)p * kTopK);
 }
 
-// rt8e256: logits = wrt . h, shared gate sg = sigmoid(wsh . h), then the top-8.  One 256-thread
-// workgroup per position; logit e is thread e's fixed-order sum (4-way split of k, then the
-// partials in order), the shared gate a fixed-order tree.
-__global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
-                                                        const float* __restrict__ h, uint16_t* __restrict__ eids,
-                                                        float* __restrict__ gates, float* __restrict__ sg) {
-  __shared__ float lg[kE];
-  __shared__ float shp[256];
-  const int p = blockIdx.x, t = threadIdx.x;
-  const float4* hr = reinterpret_cast<const float4*>(h + (size_t)p * kHid);
-  {
-    const float4* wr = reinterpret_cast<const float4*>(wrt + (size_t)t * kHid);
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int i = 0; i < kHid / 16; ++i) {
+// rt8e256: logits = wrt . h, shared gate sg = sigmoid(wsh . h), then the top-8.  A 16-wave workgroup
+// takes NP positions: their h in LDS, wave w the 16 experts 16 w .. , four lanes a row so that a
+// wave's 16-B loads read 64 contiguous bytes a quad (a row per lane, as before, took a quarter of
+// that rate), 16 or 8 loads ahead; every weight feeds NP positions.  Products and sums are fp32: 16 fixed
+// partial sums of 128 terms a logit.  The bound at few positions is the 2 MB of wrt through one
+// CU's load path (64 B a clock), at many the fp32 FMAs.
+constexpr int kRtThreads = 1024;
+template <int NP>
+__global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
+                                                               const float* __restrict__ h, uint16_t* __restrict__ eids,
+                                                               float* __restrict__ gates, float* __restrict__ sg, int P) {
+  __shared__ float4 hs[NP][kHid / 4];
+  __shared__ float4 lg[NP][kE / 4];
+  __shared__ float shp[NP][kRtThreads / TLX_WAVE];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, p0 = blockIdx.x * NP;
+  const int row = 16 * wave + (lane >> 2), piece = lane & 3;
+  constexpr int kSteps = kHid / 16;   // 16 k a step
+  constexpr int kRtAhead = NP <= 4 ? 16 : 8;   // as the sums leave room (P = 2048: 48.8 us at 16, 43.6 at 8)
+  const float4* wr = reinterpret_cast<const float4*>(wrt + (size_t)row * kHid) + piece;
+  float4 w[kRtAhead];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 w = wr[q * (kHid / 16) + i], x = hr[q * (kHid / 16) + i];
-        part[q] += w.x * x.x + w.y * x.y + w.z * x.z + w.w * x.w;
+  for (int u = 0; u < kRtAhead; ++u) w[u] = wr[4 * u];
+  for (int i = t; i < NP * (kHid / 4); i += kRtThreads) {
+    const int p = i / (kHid / 4), k4 = i % (kHid / 4);
+    hs[p][k4] = reinterpret_cast<const float4*>(h + (size_t)min(p0 + p, P - 1) * kHid)[k4];   // past P: unused
+  }
+  const float2 ws = reinterpret_cast<const float2*>(wsh)[t];
+  __syncthreads();
+  float4 acc[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) acc[p] = float4{0.f, 0.f, 0.f, 0.f};
+  // slot u of the ring: step s0 + u's weights, then (once used) step s0 + kRtAhead + u's.  The fences
+  // keep each pair of steps' requests behind its uses: without them the scheduler moves the requests
+  // to where the loop's end has to wait for all of them.
+  for (int s0 = 0; s0 < kSteps; s0 += kRtAhead) {
+    const float4* wn = wr + 4 * min(s0 + kRtAhead, kSteps - kRtAhead);   // past the end: the last steps again
+#pragma unroll
+    for (int u = 0; u < kRtAhead; ++u) {
+      const float4 wv = w[u];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const float4 x = hs[p][4 * (s0 + u) + piece];
+        acc[p].x += wv.x * x.x;
+        acc[p].y += wv.y * x.y;
+        acc[p].z += wv.z * x.z;
+        acc[p].w += wv.w * x.w;
       }
+      w[u] = wn[4 * u];
+      if (u & 1) __builtin_amdgcn_sched_barrier(0);
     }
-    lg[t] = ((part[0] + part[1]) + part[2]) + part[3];
-    const float2* ws2 = reinterpret_cast<const float2*>(wsh);
-    const float2* hr2 = reinterpret_cast<const float2*>(h + (size_t)p * kHid);
-    float s = 0.f;
+  }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float2 a = ws2[t + 256 * i], b = hr2[t + 256 * i];
-      s += a.x * b.x + a.y * b.y;
-    }
-    shp[t] = s;
+  for (int p = 0; p < NP; ++p) {
+    float v = (acc[p].x + acc[p].y) + (acc[p].z + acc[p].w);
+    v += dpp_f<0xB1, 0xF>(v);
+    v += dpp_f<0x4E, 0xF>(v);
+    if (piece == 0) reinterpret_cast<float*>(lg[p])[row] = v;
+    const float2 x = reinterpret_cast<const float2*>(hs[p])[t];
+    const float s = wave_sum(ws.x * x.x + ws.y * x.y);
+    if (lane == 0) shp[p][wave] = s;
   }
   __syncthreads();
-  for (int w = 128; w >= 1; w >>= 1) {
-    if (t < w) shp[t] += shp[t + w];
-    __syncthreads();
-  }
-  if (t < 64) {
-    float v[4];
+  if (wave < NP && p0 + wave < P) {
+    const int p = p0 + wave;
+    topk8_wave(lg[wave][lane], lane, eids + (size_t)p * kTopK, gates + (size_t)p * kTopK);
+    if (lane == 0) {
+      float s = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = lg[t + 64 * j];
-    topk8_wave(v, t, eids + (size_t)p * kTopK, gates + (size_t)p * kTopK);
-    if (t == 0) sg[p] = 1.f / (1.f + expf(-shp[0]));
+      for (int i = 0; i < kRtThreads / TLX_WAVE; ++i) s += shp[wave][i];
+      sg[p] = 1.f / (1.f + expf(-s));
+    }
   }
+}
+
+template <int NP>
+int moe_route_launch(const float* wrt, const float* wsh, const float* h, uint16_t* eids, float* gates, float* sg, int P,
+                     hipStream_t st) {
+  moe_route_kernel<NP><<<(P + NP - 1) / NP, kRtThreads, 0, st>>>(wrt, wsh, h, eids, gates, sg, P);
+  return tlx_launch_status();
 }
 
 // ------------------------------------------------------------------ sort
@@ -1151,16 +1166,24 @@ int moe_max_items(int np) { return (np + moe_item_tok(np) - 1) / moe_item_tok(np
 extern "C" int tlx_moe_topk(const float* logits, uint16_t* eids, float* gates, int P, void* stream) {
   TLX_RET_IF(P < 1, TLX_E_ARG);
   TLX_RET_IF(!tlx_aligned(logits, 16), TLX_E_ALIGN);
-  moe_topk_kernel<<<(P + 15) / 16, 256, 0, (hipStream_t)stream>>>(logits, eids, gates, P);
+  moe_topk_kernel<<<(P + 3) / 4, 256, 0, (hipStream_t)stream>>>(logits, eids, gates, P);
   return tlx_launch_status();
 }
+
+// Positions a workgroup by batch, the fewest that keep the grid within one workgroup a CU (256):
+// us at 1 / 4 / 8 positions a workgroup: P = 4 22.9 / 29.2 / 44.6, 256 24.0 / 27.7 / 45.3, 300 39.9 /
+// 27.5 / 45.3, 1024 77.9 / 29.8 / 45.6, 1500 112 / 50.2 / 45.5, 2048 148 / 57.3 / 43.6.  (A row per lane
+// and one position a workgroup: 75 us at P = 4.)
+constexpr int kRt1 = 256, kRt4 = 1024;
 
 extern "C" int tlx_moe_route(const float* wrt, const float* wsh, const float* h, uint16_t* eids, float* gates,
                              float* sg, int P, void* stream) {
   TLX_RET_IF(P < 1, TLX_E_ARG);
   TLX_RET_IF(!tlx_aligned(wrt, 16) || !tlx_aligned(h, 16) || !tlx_aligned(wsh, 8), TLX_E_ALIGN);
-  moe_route_kernel<<<P, 256, 0, (hipStream_t)stream>>>(wrt, wsh, h, eids, gates, sg);
-  return tlx_launch_status();
+  const hipStream_t st = (hipStream_t)stream;
+  if (P <= kRt1) return moe_route_launch<1>(wrt, wsh, h, eids, gates, sg, P, st);
+  if (P <= kRt4) return moe_route_launch<4>(wrt, wsh, h, eids, gates, sg, P, st);
+  return moe_route_launch<8>(wrt, wsh, h, eids, gates, sg, P, st);
 }
 
 extern "C" int tlx_moe_sort(const uint16_t* eids, int* eoff, uint16_t* plist, uint32_t* items, uint32_t* nitp,
