@@ -52,6 +52,13 @@ __device__ __forceinline__ uint32_t tlx_mix2_f16(float s, uint32_t h2) {
   return r;
 }
 
+// fp16 pairs as words: a value twice, and the products with a pair (v_pk_mul_f16, rounded once each)
+__device__ __forceinline__ _Float16 tlx_h16(uint16_t b) { return __builtin_bit_cast(_Float16, b); }
+__device__ __forceinline__ h2_t tlx_splat2(_Float16 v) { return h2_t{v, v}; }
+__device__ __forceinline__ uint32_t tlx_mul2(uint32_t a, h2_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, a) * b);
+}
+
 // An MFMA does not wait for a VALU result in its source registers: 2 wait states must separate the
 // write and the read, and the compiler inserts none after inline asm it does not look into (such as
 // the v_fma_mix above).  An operand built by tlx_mix2_f16 and read by an MFMA directly passes

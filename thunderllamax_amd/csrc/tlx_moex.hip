@@ -212,28 +212,30 @@ __device__ __forceinline__ void gv_lut_fill(GvLut& L, const float* gridf, int t)
     L.smask[t] = uint2{((t & 1u) << 15) | (((t >> 1) & 1u) << 31), (((t >> 2) & 1u) << 15) | (((t >> 3) & 1u) << 31)};
 }
 
-// The 16 weights as fp16 operands, bit for bit the fp16 of gx_decode's values: the products of a
-// block scale and an integer level are exact in f32 for all three classes (IQ3_S: fp16 d times
-// 1 + 2 nib times a level <= 15, <= 20 bits; Q8_0: d times an int8, <= 19; Q6_K: d times an int8
-// scale times q - 32, <= 23), so v_fma_mix's one rounding to fp16 is the reference's.
+// The 16 weights as fp16 operands, bit for bit the fp16 of gx_decode's values.  IQ3_S and Q8_0: packed
+// fp16 multiplies -- (1 + 2 nib) * level <= 465 and an int8 are exact fp16 integers and d is fp16 itself,
+// so the product with d is rounded once, to the reference's operand.  Q6_K: sc * (q - 32) is not exact in
+// fp16; d * sc * (q - 32) has <= 23 bits, exact in f32, and v_fma_mix rounds it once.  The multiplies
+// are the cheaper by far: 5 clocks a wave instruction for two weights against 13 for one
+// (measured: 2.6 and 6.0 ns), for IQ3_S with the second multiply 10 against 26.
 template <int CLS>
 __device__ __forceinline__ void gx_decode_h(u4_t* h, const GxRaw<CLS>& r, const GvLut* lut) {
   if constexpr (CLS == GX_IQ3S) {
-    const float db = tlx_h2f((uint16_t)(r.dn & 0xFFFFu)) * (float)(1u + 2u * (r.dn >> 16));   // exact
+    const h2_t d = tlx_splat2(tlx_h16((uint16_t)(r.dn & 0xFFFFu))), n = tlx_splat2((_Float16)(float)(1u + 2u * (r.dn >> 16)));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {   // index byte i: weights 4i .. 4i+3
       const uint2 g = lut->grid[((r.qs >> (8 * i)) & 255u) | (((r.hs >> i) & 1u) << 8)];
       const uint2 m = lut->smask[(r.hs >> (8 + 4 * i)) & 15u];
-      h[i >> 1][2 * (i & 1)] = tlx_mix2_f16(db, g.x) ^ m.x;
-      h[i >> 1][2 * (i & 1) + 1] = tlx_mix2_f16(db, g.y) ^ m.y;
+      h[i >> 1][2 * (i & 1)] = tlx_mul2(tlx_mul2(g.x, n), d) ^ m.x;
+      h[i >> 1][2 * (i & 1) + 1] = tlx_mul2(tlx_mul2(g.y, n), d) ^ m.y;
     }
   } else if constexpr (CLS == GX_Q80) {
-    const float d = tlx_h2f((uint16_t)r.d);
+    const h2_t d = tlx_splat2(tlx_h16((uint16_t)r.d));
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const uint32_t u4 = r.q[j] ^ 0x80808080u;   // int8 + 128
-      h[j >> 1][2 * (j & 1)] = tlx_mix2_f16(d, tlx_bytes_h2(u4, 0, 128.f));
-      h[j >> 1][2 * (j & 1) + 1] = tlx_mix2_f16(d, tlx_bytes_h2(u4, 1, 128.f));
+      h[j >> 1][2 * (j & 1)] = tlx_mul2(tlx_bytes_h2(u4, 0, 128.f), d);
+      h[j >> 1][2 * (j & 1) + 1] = tlx_mul2(tlx_bytes_h2(u4, 1, 128.f), d);
     }
   } else {   // Q6_K: t = d * sc, weights l = 0 .. 15 of quarter g
     const float t = tlx_h2f((uint16_t)(r.ds & 0xFFFFu)) * (float)(int8_t)(uint8_t)(r.ds >> 16);
@@ -536,15 +538,16 @@ __device__ __forceinline__ int gv_koff(int kq, int s) {
 template <int CLS, int S>
 __device__ __forceinline__ h8_t gv_decode(const GvRaw<CLS>& r, int kq, const GvLut* lut) {
   if constexpr (CLS == GX_IQ3S) {
-    const float db = tlx_h2f((uint16_t)(r.dq & 0xFFFFu)) * (float)(1u + 2u * ((r.sc >> (4 * (S >> 2))) & 15u));
+    const h2_t d = tlx_splat2(tlx_h16((uint16_t)(r.dq & 0xFFFFu)));
+    const h2_t n = tlx_splat2((_Float16)(float)(1u + 2u * ((r.sc >> (4 * (S >> 2))) & 15u)));
     const uint32_t qsw = r.qs[S >> 1] >> (16 * (S & 1));
     const uint32_t qh = r.dq >> (16 + 2 * S);
     const uint2 g0 = lut->grid[(qsw & 255u) | ((qh & 1u) << 8)];
     const uint2 g1 = lut->grid[((qsw >> 8) & 255u) | ((qh & 2u) << 7)];
     const uint32_t sb = (S < 4 ? r.sg0 : r.sg1) >> (8 * (S & 3));
     const uint2 m0 = lut->smask[sb & 15u], m1 = lut->smask[(sb >> 4) & 15u];
-    // (each word's last write is the sign XOR, an instruction the compiler sees: no guard needed)
-    const u4_t h = {tlx_mix2_f16(db, g0.x) ^ m0.x, tlx_mix2_f16(db, g0.y) ^ m0.y, tlx_mix2_f16(db, g1.x) ^ m1.x, tlx_mix2_f16(db, g1.y) ^ m1.y};
+    const u4_t h = {tlx_mul2(tlx_mul2(g0.x, n), d) ^ m0.x, tlx_mul2(tlx_mul2(g0.y, n), d) ^ m0.y,
+                    tlx_mul2(tlx_mul2(g1.x, n), d) ^ m1.x, tlx_mul2(tlx_mul2(g1.y, n), d) ^ m1.y};
     return __builtin_bit_cast(h8_t, h);
   } else if constexpr (CLS == GX_Q6K) {
     constexpr int n = S >> 2, q = S & 3;
@@ -564,15 +567,14 @@ __device__ __forceinline__ h8_t gv_decode(const GvRaw<CLS>& r, int kq, const GvL
   } else {
     constexpr int blk = S >> 2, q = S & 3;
     const u4_t& qv = blk ? ((q < 2) ? r.q2 : r.q3) : ((q < 2) ? r.q0 : r.q1);
-    const float d = tlx_h2f((uint16_t)(r.d >> (16 * blk)));
+    const h2_t d = tlx_splat2(tlx_h16((uint16_t)(r.d >> (16 * blk))));
     u4_t h;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint32_t u4 = qv[2 * (q & 1) + j] ^ 0x80808080u;   // int8 + 128
-      h[2 * j] = tlx_mix2_f16(d, tlx_bytes_h2(u4, 0, 128.f));
-      h[2 * j + 1] = tlx_mix2_f16(d, tlx_bytes_h2(u4, 1, 128.f));
+      h[2 * j] = tlx_mul2(tlx_bytes_h2(u4, 0, 128.f), d);
+      h[2 * j + 1] = tlx_mul2(tlx_bytes_h2(u4, 1, 128.f), d);
     }
-    tlx_mfma_operand_guard(h);
     return __builtin_bit_cast(h8_t, h);
   }
 }
