@@ -37,19 +37,24 @@ __device__ __forceinline__ uint16_t tlx_f2h_bits(float f) {
   return __builtin_bit_cast(uint16_t, (_Float16)f);
 }
 
-// fp16 pair {s * lo(h2), s * hi(h2)}: v_fma_mix takes the two fp16 halves of h2 as operands and
-// rounds each product to fp16 once, from the exact value (measured: 1 + 2^-11 + 2^-40 gives
-// 1 + 2^-10, not the 1.0 an intermediate f32 rounding would).  So it is the reference's fp16(f32
-// product) bit for bit only where the product is exact in f32 -- a block scale of <= 18
-// significant bits (fp16 d times a small integer) times a level of <= 6 -- and is not used for
-// a*q - b forms (Q4_K / Q5_K), whose f32 result can round.
-__device__ __forceinline__ uint32_t tlx_mix2_f16(float s, uint32_t h2) {
+// fp16 pair {lo, hi} of two f32 values, each rounded to nearest even (one instruction; from separate
+// conversions the compiler makes three)
+__device__ __forceinline__ uint32_t tlx_pack2_f16(float lo, float hi) {
   uint32_t r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]\n\t"
-      "v_fma_mixhi_f16 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]"
-      : "=&v"(r)
-      : "v"(s), "v"(h2));
+  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
   return r;
+}
+
+// fp16 pair {s * lo(h2), s * hi(h2)}: two f32 products with the halves of h2 as operands, then one
+// conversion of both.  It is the reference's fp16(f32 product) bit for bit; where the product is exact
+// in f32 -- a block scale of <= 18 significant bits (fp16 d times a small integer) times a level of
+// <= 6 -- also fp16 of the exact value.  (v_fma_mixlo / mixhi write a half each, the second waiting for
+// the first, at half rate: measured 12 ns a pair and SIMD, this 6.7.)
+__device__ __forceinline__ uint32_t tlx_mix2_f16(float s, uint32_t h2) {
+  float lo, hi;
+  asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(lo) : "v"(s), "v"(h2));
+  asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(hi) : "v"(s), "v"(h2));
+  return tlx_pack2_f16(lo, hi);
 }
 
 // fp16 pairs as words: a value twice, and the products with a pair (v_pk_mul_f16, rounded once each)
@@ -61,7 +66,7 @@ __device__ __forceinline__ uint32_t tlx_mul2(uint32_t a, h2_t b) {
 
 // An MFMA does not wait for a VALU result in its source registers: 2 wait states must separate the
 // write and the read, and the compiler inserts none after inline asm it does not look into (such as
-// the v_fma_mix above).  An operand built by tlx_mix2_f16 and read by an MFMA directly passes
+// the conversion above).  An operand built by tlx_mix2_f16 and read by an MFMA directly passes
 // through this guard first: its nops sit after the operand's last write (the asm takes the operand
 // as an input) and before the MFMA (which takes it as an output).
 __device__ __forceinline__ void tlx_mfma_operand_guard(u4_t& h) { asm volatile("s_nop 2" : "+v"(h)); }

@@ -274,12 +274,6 @@ __device__ __forceinline__ void pf_kq_read(PfKq& r, const PfLds& L, int stage, i
   }
 }
 
-// fp16 of an fp32 value, round to nearest even (the reference's __float2half)
-__device__ __forceinline__ uint32_t pf_pack2(float a, float b) {
-  const h2_t v = {(_Float16)a, (_Float16)b};
-  return __builtin_bit_cast(uint32_t, v);
-}
-
 // The 16 operand values of sub-block j for half h into pieces 2h, 2h + 1 of tile row r.
 template <int FMT>
 __device__ __forceinline__ void pf_kq_dequant(const PfKq& r, _Float16* bt, int row, int j, int h) {
@@ -310,12 +304,11 @@ __device__ __forceinline__ void pf_kq_dequant(const PfKq& r, _Float16* bt, int r
       float f[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[e] = __builtin_fmaf(A, (float)((qv >> (8 * e)) & 0xFFu), -B);
-      w[2 * i] = pf_pack2(f[0], f[1]);
-      w[2 * i + 1] = pf_pack2(f[2], f[3]);
+      w[2 * i] = tlx_pack2_f16(f[0], f[1]);
+      w[2 * i + 1] = tlx_pack2_f16(f[2], f[3]);
     }
   } else {
-    // A * (q - 32) has at most 11 + 7 + 5 = 23 significant bits: exact in f32, so v_fma_mix's
-    // one rounding of the product (the level as an fp16 integer) is fp16(f32 product)
+    // A * (q - 32), the level as an fp16 integer: at most 11 + 7 + 5 = 23 significant bits, exact in f32
     const int hp = s >> 2, g = s & 3;
     const float d = tlx_h2f((uint16_t)r.hdr.x);
     const int sci = (8 * hp + h + 2 * g) & 3;
