@@ -148,3 +148,51 @@ def test_pfg3_bad_arguments_raise(gpu):
         ops.pfg3_iq3o(w, g, torch.zeros(256, 320, dtype=torch.float16, device=gpu), out)
     with pytest.raises(TlxError):   # N not a multiple of the 256-row tile
         ops.pfg3_iq3o(w, g, x, torch.empty(256, 128, dtype=torch.float16, device=gpu))
+
+
+def _units(gpu, seed, rows, kdim):
+    """packed7 units of seeded IQ3_XXS rows, repacked on the GPU."""
+    g = torch.Generator(device=gpu)
+    g.manual_seed(seed)
+    w = torch.randint(0, 256, (rows, 98 * (kdim // 256)), dtype=torch.uint8, device=gpu, generator=g)
+    w[:, 96 * (kdim // 256):] = 0x14   # d (the packed rows' last field): fp16 1.22e-3
+    return ops.pack_w7(w, torch.empty(rows * kdim // 2, dtype=torch.uint8, device=gpu), rows, kdim)
+
+
+@pytest.mark.parametrize("M,N,K,mib", [
+    (256, 5120, 17408, 128),    # 20 tiles: ranges that divide a tile (12 each)
+    (256, 5120, 17408, 11),     # the same with room for 44 parts: one range fewer or none
+    (512, 256, 4096, 128),      # 2 tiles of 32 chunks, at least 4 chunks a range
+    (2048, 5120, 2304, 128),    # 160 tiles of 18 chunks in 256 ranges: two segments a workgroup
+    (256, 17408 * 2, 5120, 128),   # 136 tiles of 40 chunks: two segments a workgroup
+])
+def test_pfg3_split_ranges(gpu, M, N, K, mib):
+    """The split schedules against whole tiles (no workspace): the same products in another fp32 order
+    (at most K roundings of 2^-24 of the row's norm-wise sum: 1e-5 holds), every output written, and the
+    same bits on every call."""
+    print(f"[case] pfg3 split M={M} N={N} K={K} workspace {mib} MiB", flush=True)
+    grid = formats.gridf_tensor(gpu)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(M + N + K)
+    x = torch.randn(M, K, device=gpu, generator=g).half()
+    res = torch.randn(M, N, device=gpu, generator=g)
+    w = _units(gpu, 1, N, K)
+    outs = []
+    try:
+        for size in (0, mib << 20, mib << 20):
+            ops.attach_workspace(gpu, gemm_bytes=size)
+            y = torch.full((M, N), float("nan"), device=gpu)
+            ops.pfg3_iq3d(w, grid, x, res, y)
+            ffn = torch.full((M, N // 2), float("nan"), dtype=torch.float16, device=gpu)
+            ops.pfg3_ffn(w[:w.numel() // 2], w[w.numel() // 2:], grid, x, ffn)
+            torch.cuda.synchronize()
+            outs.append((y, ffn))
+    finally:
+        ops.attach_workspace(gpu)
+    (whole, fw), (split, fs), (again, fa) = outs
+    assert torch.equal(split, again) and torch.equal(fs.view(torch.int16), fa.view(torch.int16))
+    err = ((split - whole).double().norm(dim=1) / (whole - res).double().norm(dim=1)).max().item()
+    assert err <= 1e-5, err
+    # the fp16 SwiGLU of sums that differ by 1e-5: a few outputs move by one fp16 rounding (2^-11)
+    errf = ((fs.double() - fw.double()).norm() / fw.double().norm()).item()
+    assert errf <= 2.0 ** -11, errf

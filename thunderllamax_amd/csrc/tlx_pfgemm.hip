@@ -47,6 +47,7 @@
 #include "tlx_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -401,17 +402,24 @@ __device__ __forceinline__ void pf_kq_step(PfLds& L, f4_t (&acc)[kMI][8], const 
 }
 
 // Schedule: `full` workgroups own one whole tile each (the complete rounds of one workgroup per
-// CU); the remaining r tiles are split into p chunk ranges (segments) whose workgroups fill the
-// last round(s).  Segments store their fp32 parts; pf_fix_kernel sums each split tile's parts in
-// segment order.  (Combining inside the kernel -- last arriver adds -- needs the parts visible
-// across the XCDs' L2s: per-access coherent atomics or agent-scope fences on ~1 MB per tile cost
-// more than the split saved.)  Tile index tau maps to (m-tile, n-tile) so that, when there are m-tiles for all 8
-// XCDs, workgroup tau runs on XCD tau % 8 and each XCD sweeps the n-tiles of its m-tiles, keeping
-// that activation slice in its L2.
+// CU); the k-chunks of the remaining r tiles, tile after tile, are cut into G equal ranges, one per
+// workgroup of the last round.  A range is no longer than a tile (G > r), so it touches at most two:
+// its workgroup computes them one after the other as segments and stores each one's fp32 part in
+// slot 2 g or 2 g + 1; pf_fix_kernel sums a tile's parts in range order.  (Combining inside the kernel
+// -- last arriver adds -- needs the parts visible across the XCDs' L2s: per-access coherent atomics or
+// agent-scope fences on ~1 MB per tile cost more than the split saved.)  Tile index tau maps to
+// (m-tile, n-tile) so that, when there are m-tiles for all 8 XCDs, workgroup tau runs on XCD tau % 8
+// and each XCD sweeps the n-tiles of its m-tiles, keeping that activation slice in its L2.
 struct PfSk {
-  int full, r, p;      // whole-tile workgroups, split tiles, segments per split tile
-  float* part;         // workspace: one 256 KB fp32 slot per segment
+  int full, r, G;      // whole-tile workgroups, split tiles, ranges
+  float* part;         // workspace: two 256 KB fp32 slots per range
 };
+
+// first chunk of range g (counted over the split tiles' chunks), and the range that holds chunk c
+__host__ __device__ __forceinline__ int pf_range_lo(int chunks, int G, int g) { return (int)((int64_t)chunks * g / G); }
+__host__ __device__ __forceinline__ int pf_range_of(int chunks, int G, int c) {
+  return (int)(((int64_t)(c + 1) * G + chunks - 1) / chunks) - 1;
+}
 
 template <int EPI>
 __device__ __forceinline__ void pf_epilogue(const f4_t (&acc)[kMI][8], const int* bg, int m0, int nt, int wm, int kq,
@@ -553,19 +561,22 @@ __global__ __launch_bounds__(kThreads, 1) void pf_gemm_kernel(
   __shared__ PfLds L;
   const int nch = K / 128;
   const int bx = (int)blockIdx.x;
-  int tau, h0 = 0, h1 = nch, seg = -1;
-  if (bx < sk.full) {
-    tau = bx;
-  } else {
-    seg = bx - sk.full;
-    const int q = seg % sk.p;
-    tau = sk.full + seg / sk.p;
-    h0 = q * nch / sk.p;
-    h1 = (q + 1) * nch / sk.p;
-  }
   int mt, nt;
-  pf_tile_of(tau, mtiles, ntiles, mt, nt);
-  pf_tile<EPI, PF_IQ3>(L, w1, w2, nullptr, gridf, x, out, res, N, K, mt, nt, h0, h1, seg, sk);
+  if (bx < sk.full) {
+    pf_tile_of(bx, mtiles, ntiles, mt, nt);
+    pf_tile<EPI, PF_IQ3>(L, w1, w2, nullptr, gridf, x, out, res, N, K, mt, nt, 0, nch, -1, sk);
+    return;
+  }
+  // a range's chunks [u, u1) counted over the split tiles
+  const int g = bx - sk.full, u1 = pf_range_lo(sk.r * nch, sk.G, g + 1);
+  int u = pf_range_lo(sk.r * nch, sk.G, g);
+  for (int slot = 2 * g; u < u1; ++slot) {
+    const int st = u / nch, h0 = u - st * nch, h1 = min(nch, h0 + (u1 - u));
+    pf_tile_of(sk.full + st, mtiles, ntiles, mt, nt);
+    if (slot & 1) __syncthreads();   // the first segment's LDS is free in every wave
+    pf_tile<EPI, PF_IQ3>(L, w1, w2, nullptr, gridf, x, out, res, N, K, mt, nt, h0, h1, slot, sk);
+    u += h1 - h0;
+  }
 }
 
 // The merged form: up to three segments (matrices of any PfFmt sharing x), fp16 outputs; the
@@ -592,7 +603,7 @@ __global__ __launch_bounds__(kThreads, 1) void pfm_gemm_kernel(const PfMulti mse
   while (s + 1 < mseg.nseg && ntg >= mseg.seg[s + 1].nt0) ++s;
   const PfSeg sg = mseg.seg[s];
   const int nt = ntg - sg.nt0, nch = K / 128;
-  const PfSk none{0, 0, 1, nullptr};
+  const PfSk none{0, 0, 0, nullptr};
   const u4_t* w = static_cast<const u4_t*>(sg.w);
   const uint8_t* wb = static_cast<const uint8_t*>(sg.w);
   switch (sg.fmt) {
@@ -610,44 +621,61 @@ int pf_check(const void* w, const void* x, int M, int N, int K, int layout, int 
   return TLX_OK;
 }
 
-// The split tiles' sums: workgroup (st, i) adds the p parts of row group i (16 rows per wave
-// row) of split tile st in segment order (fixed: the result does not depend on which segment
-// finished first) and applies the epilogue to them.  8 workgroups a tile keep the reads spread.
+// The split tiles' sums: workgroup (st, i, jp) adds the parts of row group i (16 rows per wave row) and
+// column groups jp, jp + 4 of split tile st in range order (fixed: the result does not depend on which
+// range finished first) and applies the epilogue to them.  Bound by the parts' bytes: 16 workgroups a
+// tile, each thread's loads of up to four parts in flight (8 workgroups with one part at a time in
+// flight: M = 256 down 21 us for 21 MB).
+constexpr int kFixPer = 4 * kMI;
 template <int EPI>
-__global__ __launch_bounds__(kThreads) void pf_fix_kernel(const f4_t* __restrict__ part, void* __restrict__ out,
-                                                          const float* __restrict__ res, int N, int mtiles,
-                                                          int ntiles, int full, int p) {
+__global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out, const float* __restrict__ res, int N, int nch,
+                                                          int mtiles, int ntiles, const PfSk sk) {
   constexpr bool kFfn = EPI == PF_FFN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int col = lane & 15, kq = lane >> 4, wm = wave >> 1, wn = wave & 1;
-  const int st = (int)blockIdx.x / kMI, i = (int)blockIdx.x % kMI, tau = full + st;
+  const int st = (int)blockIdx.x / kFixPer, i = (int)blockIdx.x % kFixPer >> 2, jp = (int)blockIdx.x & 3;
   int mt, nt;
-  pf_tile_of(tau, mtiles, ntiles, mt, nt);
-  int bg[8];
+  pf_tile_of(sk.full + st, mtiles, ntiles, mt, nt);
+  const int chunks = sk.r * nch, c0 = st * nch;
+  const int g0 = pf_range_of(chunks, sk.G, c0), g1 = pf_range_of(chunks, sk.G, c0 + nch - 1);
+  constexpr size_t kSlot = kBM * kBN / 4;
+  const f4_t* part = reinterpret_cast<const f4_t*>(sk.part) + (size_t)(i * 8 + jp) * kThreads + threadIdx.x;
+  // range g0 may have begun in the tile before: this tile is then its second segment
+  const int s0 = 2 * g0 + (pf_range_lo(chunks, sk.G, g0) < c0 ? 1 : 0);
+  f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+  const auto add = [&](auto count, int g) {   // parts g .. g + count - 1, all requested first
+    constexpr int C = decltype(count)::value;
+    f4_t v[C][2];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) bg[j] = kFfn ? (j < 4 ? 4 * wn + j : 8 + 4 * wn + (j - 4)) : 8 * wn + j;
-  f4_t acc[8];
-  const f4_t* src = part + (size_t)st * p * (kBM * kBN / 4) + i * 8 * kThreads + threadIdx.x;
+    for (int q = 0; q < C; ++q) {
+      const f4_t* p = part + (size_t)(g + q == g0 ? s0 : 2 * (g + q)) * kSlot;
+      v[q][0] = p[0];
+      v[q][1] = p[4 * kThreads];
+    }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    f4_t sum = src[j * kThreads];
-    for (int q = 1; q < p; ++q) sum += src[(size_t)q * (kBM * kBN / 4) + j * kThreads];
-    acc[j] = sum;
+    for (int q = 0; q < C; ++q) {
+      acc[0] += v[q][0];
+      acc[1] += v[q][1];
+    }
+  };
+  int g = g0;
+  for (; g + 3 <= g1; g += 4) add(std::integral_constant<int, 4>{}, g);
+  switch (g1 - g + 1) {
+    case 3: add(std::integral_constant<int, 3>{}, g); break;
+    case 2: add(std::integral_constant<int, 2>{}, g); break;
+    case 1: add(std::integral_constant<int, 1>{}, g); break;
+    default: break;
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int m = mt * kBM + 16 * kMI * wm + 16 * i + 4 * kq + e;
-    if constexpr (EPI == PF_FFN) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = nt * (kBN / 2) + 16 * bg[j] + col;
-        reinterpret_cast<uint16_t*>(out)[(size_t)m * N + n] = tlx_swiglu_bits(acc[j][e], acc[j + 4][e]);
-      }
+    if constexpr (kFfn) {   // column groups: gate 4 wn + jp, up 8 + 4 wn + jp
+      const int n = nt * (kBN / 2) + 16 * (4 * wn + jp) + col;
+      reinterpret_cast<uint16_t*>(out)[(size_t)m * N + n] = tlx_swiglu_bits(acc[0][e], acc[1][e]);
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int n = nt * kBN + 16 * bg[j] + col;
-        const size_t o = (size_t)m * N + n;
+      for (int j = 0; j < 2; ++j) {
+        const size_t o = (size_t)m * N + nt * kBN + 16 * (8 * wn + jp + 4 * j) + col;
         if constexpr (EPI == PF_RES)
           reinterpret_cast<float*>(out)[o] = res[o] + acc[j][e];
         else
@@ -657,38 +685,47 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(const f4_t* __restrict
   }
 }
 
-// Launch shape: whole tiles for the complete rounds of one workgroup per CU; the r tiles left
-// over are split into p segments, p (<= 4) minimizing the chunks the busiest CU computes
-// (ties: fewer segments), when that beats one more round of whole tiles.
+// Launch shape: whole tiles for the complete rounds of one workgroup per CU; the chunks of the r tiles
+// left over in G ranges, G one a CU or the multiples of r (every range inside a tile: one segment a
+// workgroup, fewer parts), as far as the workspace's slots go.  The G of least cost, where that beats
+// one more round of whole tiles.  Cost in 1/40 chunk (0.1 us; a 128-k chunk of a tile takes about 4 us a
+// CU): the longest range's chunks, 1.5 chunks a segment for its prologue, 1 a part (256 KB written and
+// read again).  Measured, the FFN block (G by equal splits of 2 to 4 a tile -> by this rule): M = 256
+// 284 -> 198 us (down: 80 workgroups -> 240).  With G always one a CU M = 1536 took 873 us against 862.
+int pf_ranges(int r, int nch, int G0, int64_t slots) {
+  const int64_t chunks = (int64_t)r * nch;
+  int best = 0;
+  int64_t least = 40LL * nch;
+  const auto take = [&](int64_t G, int64_t segs, int64_t parts, int64_t need) {
+    if (G <= r || 4 * G > chunks || need > slots) return;
+    const int64_t cost = 40 * ((chunks + G - 1) / G) + 60 * segs + parts;
+    if (cost < least) { least = cost; best = (int)G; }
+  };
+  for (int64_t G = 2 * (int64_t)r; G <= G0; G += r) take(G, 1, G, 2 * G);
+  take(G0, 2, r + G0 - 1, 2 * (int64_t)G0);
+  return best;
+}
+
 template <int EPI>
 int pf_launch(const u4_t* w1, const u4_t* w2, const float* gridf, const _Float16* x, void* out, const float* res,
               int M, int N, int K, int mtiles, int ntiles, hipStream_t st) {
   const int tiles = mtiles * ntiles, G0 = tlx_cu_count(), nch = K / 128;
   const int R = tiles / G0, r = tiles - R * G0;
-  PfSk sk{tiles, 0, 1, nullptr};
+  PfSk sk{tiles, 0, 0, nullptr};
   if (r > 0) {
-    // the split needs r * p parts of 256 KB in the attached workspace; without room, whole tiles
     void* ws = nullptr;
     size_t wsb = 0;
     const int rc = tlx_workspace_gemm(&ws, &wsb);
     TLX_RET_IF(rc != TLX_OK, rc);
-    const size_t cap = ws != nullptr ? std::min(wsb, kPfPartBytes) : 0;
-    int best_p = 1;
-    long best = (long)(R + 1) * nch;
-    for (int p = 2; p <= 4; ++p) {
-      if ((size_t)r * p * (kBM * kBN * 4) > cap || r > kPfMaxTiles) break;
-      const long span = (long)R * nch + (long)((r * p + G0 - 1) / G0) * ((nch + p - 1) / p);
-      if (span < best) { best = span; best_p = p; }
-    }
-    if (best_p > 1) sk = PfSk{R * G0, r, best_p, static_cast<float*>(ws)};
+    const int64_t slots = ws != nullptr ? (int64_t)(std::min(wsb, kPfPartBytes) / (kBM * kBN * 4)) : 0;
+    const int G = pf_ranges(r, nch, G0, slots);
+    if (G > 0) sk = PfSk{R * G0, r, G, static_cast<float*>(ws)};
   }
-  pf_gemm_kernel<EPI><<<sk.full + sk.r * sk.p, kThreads, 0, st>>>(w1, w2, gridf, x, out, res, M, N, K, mtiles,
-                                                                    ntiles, sk);
-  if (sk.p > 1) {
+  pf_gemm_kernel<EPI><<<sk.full + sk.G, kThreads, 0, st>>>(w1, w2, gridf, x, out, res, M, N, K, mtiles, ntiles, sk);
+  if (sk.G > 0) {
     const int rc = tlx_launch_status();
     TLX_RET_IF(rc != TLX_OK, rc);
-    pf_fix_kernel<EPI><<<sk.r * kMI, kThreads, 0, st>>>(reinterpret_cast<const f4_t*>(sk.part), out, res, N, mtiles,
-                                                      ntiles, sk.full, sk.p);
+    pf_fix_kernel<EPI><<<sk.r * kFixPer, kThreads, 0, st>>>(out, res, N, nch, mtiles, ntiles, sk);
   }
   return tlx_launch_status();
 }
