@@ -349,3 +349,33 @@ def test_attention_variants(gpu, name, M):
     errs = _attn_case(gpu, name, M, 600 + M)
     print(f"[{name} M={M}] q/k/v rel-err {errs}")
     assert max(errs) <= TOL
+
+
+# Edges of the one-launch Q6_K / IQ3_XXS / Q4_K projection: fewer blocks than waves and a block count
+# that 8 waves do not divide, tail tiles, several tiles a workgroup in each matrix (more tiles than
+# CUs), a matrix of one tile, and row counts around the row group of K = 5120 (12 rows).
+@pytest.mark.parametrize("K,Nq,Nk,Nv,M,v4,raw", [
+    (512, 4009, 250, 1003, 3, True, False), (512, 16, 4500, 9, 16, False, False),
+    (2560, 100, 17, 5000, 7, True, True), (5120, 33, 40, 24, 12, True, False),
+    (5120, 33, 40, 24, 13, False, False), (256, 16, 16, 16, 1, True, True)])
+def test_qkv_three_formats_one_launch(gpu, K, Nq, Nk, Nv, M, v4, raw):
+    from thunderllamax_amd._lib import V_Q4K
+    print(f"[case] q6/iq3/q4 K={K} rows {Nq} {Nk} {Nv} M={M} v4={v4} raw={raw}", flush=True)
+    rng = np.random.default_rng(K + Nq + M)
+    deq3 = lambda r: quants.dequant_iq3xxs_blocks(r.reshape(-1, 98)).reshape(len(r), K)
+    rq, rk = synth.q6k_raw(rng, Nq, K), synth.iq3xxs_raw(rng, Nk, K)
+    rv = synth.k4_raw(rng, Nv, K, False) if v4 else synth.iq3xxs_raw(rng, Nv, K)
+    W = (quants.dequant_q6k(rq, K), deq3(rk), quants.dequant_q4k(rv, K) if v4 else deq3(rv))
+    x = synth.activations_f16(rng, M, K)
+    if raw:
+        w, fn = (rq, rk, rv), ops.a_qkv_q6
+    else:
+        w = (rq, formats.iq3_pack_rows(rk, K), rv if v4 else formats.iq3_pack_rows(rv, K))
+        fn = lambda *a: ops.aq6k8(*a, layout=LAYOUT_RAW | (V_Q4K if v4 else 0))
+    outs = [torch.full((M, n), float("nan"), dtype=torch.float16, device=gpu) for n in (Nq, Nk, Nv)]
+    fn(*[torch.from_numpy(np.ascontiguousarray(t)).to(gpu) for t in w], formats.gridf_tensor(gpu),
+       torch.from_numpy(x).to(gpu), *outs)
+    torch.cuda.synchronize()
+    errs = [_rows_err(o.cpu().numpy(), gemv.gemv16_ref(Wm, x)[1]) for o, Wm in zip(outs, W)]
+    print(f"[q6/iq3/q4 K={K} M={M}] q/k/v rel-err {errs}")
+    assert max(errs) <= TOL

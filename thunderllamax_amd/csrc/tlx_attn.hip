@@ -1,7 +1,7 @@
 // Fused attention q/k/v projections: the reference's four warp-range kernels (aq3k8, aq6k8,
-// a_qkv_iq3, a_qkv_q6) as one entry point each.  Segments of one quant format share a launch;
-// a segment in another format (the Q6_K q, the Q4_K v) takes a launch of its own on the same
-// stream.  Every argument is validated before anything is launched.
+// a_qkv_iq3, a_qkv_q6) as one entry point each.  A Q6_K q, its k and its v share one launch
+// (tlx_kq_mix); with an IQ3_XXS q the IQ3_XXS segments share a launch and a Q4_K v takes one of
+// its own on the same stream.  Every argument is validated before anything is launched.
 #include "tlx_common.h"
 
 namespace {
@@ -28,15 +28,18 @@ int attn_iq3(const void* wq, const void* wk, const void* wv, const float* gridf,
 int attn_q6(int fmt, const void* wq, const void* wk, const void* wv, const float* gridf,
             const uint16_t* xh, uint16_t* qrow, uint16_t* krow, uint16_t* vrow, int M, int Nq,
             int Nk, int Nv, int K, int klayout, bool v4, void* stream) {
-  const void* w[2] = {wk, wv};
-  uint16_t* out[2] = {krow, vrow};
-  const int n[2] = {Nk, Nv};
+  const void* w[3] = {wq, wk, wv};
+  uint16_t* out[3] = {qrow, krow, vrow};
+  const int n[3] = {Nq, Nk, Nv};
   const int nseg = v4 ? 1 : 2;
   int rc = tlx_kq_gemv(fmt, wq, xh, qrow, M, Nq, K, false, stream);
-  if (rc == TLX_OK) rc = tlx_iq3_segments(w, out, n, nseg, gridf, xh, M, K, klayout, false, stream);
+  if (rc == TLX_OK) rc = tlx_iq3_segments(w + 1, out + 1, n + 1, nseg, gridf, xh, M, K, klayout, false, stream);
   if (rc == TLX_OK && v4) rc = tlx_kq_gemv(kQ4K, wv, xh, vrow, M, Nv, K, false, stream);
   TLX_RET_IF(rc != TLX_OK, rc);
-  rc = tlx_iq3_segments(w, out, n, nseg, gridf, xh, M, K, klayout, true, stream);
+  bool done = false;
+  rc = tlx_kq_mix(fmt, w, out, n, gridf, xh, M, K, klayout == TLX_LAYOUT_RAW, v4, &done, stream);
+  TLX_RET_IF(done || rc != TLX_OK, rc);
+  rc = tlx_iq3_segments(w + 1, out + 1, n + 1, nseg, gridf, xh, M, K, klayout, true, stream);
   if (rc == TLX_OK && v4) rc = tlx_kq_gemv(kQ4K, wv, xh, vrow, M, Nv, K, true, stream);
   if (rc == TLX_OK) rc = tlx_kq_gemv(fmt, wq, xh, qrow, M, Nq, K, true, stream);
   return rc;

@@ -126,6 +126,17 @@ __device__ __forceinline__ void tlx_iq3_table(u2_t* tbl, const float* __restrict
     tlx_iq3_table_entries(tbl, reinterpret_cast<const float4*>(gridf)[e & 255], e & 255, e >> 8);
 }
 
+// 8 signed grid magnitudes of one lane-chunk: q word = two grid indices, sidx = the 7-bit
+// sign field; the 8th sign is the parity of sidx.
+__device__ __forceinline__ h8_t tlx_iq3_chunk(const u2_t* tbl, uint32_t qw, uint32_t sidx) {
+  const uint32_t par = __builtin_popcount(sidx) & 1u;
+  const uint32_t i0 = ((sidx & 0xFu) << 8) | (qw & 0xFFu);
+  const uint32_t i1 = (((sidx >> 4) | (par << 3)) << 8) | ((qw >> 8) & 0xFFu);
+  const u2_t a = tbl[i0];
+  const u2_t b = tbl[i1];
+  return __builtin_bit_cast(h8_t, u4_t{a.x, a.y, b.x, b.y});
+}
+
 // ---------------------------------------------------------------- device properties
 // Compute-unit count of the current device (tlx_core.hip; cached per device, one cache for the
 // whole library, filled at the latest by tlx_attach_workspace).
@@ -167,7 +178,6 @@ int tlx_workspace(void** ws);
 // The prefill GEMM's split-tile workspace: fp32 parts of 256 x 256 tiles (256 KB each), caller
 // owned and attached per device like the GEMV workspace; without one (or when it is too small for
 // a split) the GEMM runs whole tiles only.
-constexpr int kPfMaxTiles = 65536;
 constexpr size_t kPfPartBytes = size_t(512) * 256 * 256 * 4;
 constexpr size_t kPfWsBytes = kPfPartBytes;
 int tlx_workspace_gemm(void** ws, size_t* bytes);
@@ -190,5 +200,9 @@ int tlx_iq3s_launch(int nmat, int epi, int nseg, const void* const* w, const voi
 //   k-quants: fmt 0 = Q6_K raw, 1 = Q6_K padded, 2 = Q4_K, 3 = Q5_K (tlx_kquant.hip).
 //   one-time kernel set-up of the k-quant GEMVs (dynamic LDS limit), run by tlx_attach_workspace
 int tlx_kq_setup();
+// One launch over a Q6_K q (fmt), an IQ3_XXS k and a Q4_K (v4) or IQ3_XXS v, arguments checked by
+// the caller; *done is false, and nothing is launched, where separate launches are the better form.
+int tlx_kq_mix(int fmt, const void* const* w, uint16_t* const* out, const int* n, const float* gridf,
+               const uint16_t* x_f16, int M, int K, bool kraw, bool v4, bool* done, void* stream);
 int tlx_kq_gemv(int fmt, const void* w, const uint16_t* x_f16, uint16_t* out_f16, int M, int N,
                 int K, bool launch, void* stream);

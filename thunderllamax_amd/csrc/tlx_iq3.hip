@@ -33,17 +33,6 @@ constexpr int kXtMinM = 6;  // from this M on, activations are read from the til
 
 enum Epi { EPI_F16 = 0, EPI_SWIGLU = 1, EPI_RESID = 2 };
 
-// 8 signed grid magnitudes of one lane-chunk: q word = two grid indices, sidx = the 7-bit
-// sign field; the 8th sign is the parity of sidx.
-__device__ __forceinline__ h8_t iq3_chunk(const u2_t* tbl, uint32_t qw, uint32_t sidx) {
-  const uint32_t par = __builtin_popcount(sidx) & 1u;
-  const uint32_t i0 = ((sidx & 0xFu) << 8) | (qw & 0xFFu);
-  const uint32_t i1 = (((sidx >> 4) | (par << 3)) << 8) | ((qw >> 8) & 0xFFu);
-  const u2_t a = tbl[i0];
-  const u2_t b = tbl[i1];
-  return __builtin_bit_cast(h8_t, u4_t{a.x, a.y, b.x, b.y});
-}
-
 __device__ __forceinline__ h8_t splat8(_Float16 v) { return h8_t{v, v, v, v, v, v, v, v}; }
 
 struct Iq3Seg {
@@ -184,7 +173,7 @@ __global__ __launch_bounds__(WAVES * TLX_WAVE) void iq3_gemv_kernel(const Iq3Lau
         const uint32_t qw = (t & 1) ? (qd >> 16) : (qd & 0xFFFFu);
         const uint32_t sw = (t < 4) ? cur.sw[i].x : cur.sw[i].y;
         const uint32_t sidx = (sw >> (7 * (t & 3))) & 0x7Fu;
-        const h8_t B = iq3_chunk(tbl, qw, sidx) * splat8(t < 4 ? ks0 : ks1);
+        const h8_t B = tlx_iq3_chunk(tbl, qw, sidx) * splat8(t < 4 ? ks0 : ks1);
         D = __builtin_amdgcn_mfma_f32_16x16x32_f16(X[t], B, D, 0, 0, 0);
       }
       const float d = tlx_h2f((uint16_t)cur.d[i]);

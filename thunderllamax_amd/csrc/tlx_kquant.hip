@@ -26,6 +26,7 @@
 //     through LDS in wave order after the main loop, so results do not depend on scheduling.
 #include "tlx_common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace {
@@ -236,9 +237,9 @@ __host__ __device__ inline size_t k_lds_bytes(int F, int M, int K) {
          (size_t)kWaves * 16 * kgeo(F).rs;
 }
 
+// Workgroup `bid` of a launch over one matrix.
 template <int F>
-__global__ __launch_bounds__(kWaves * TLX_WAVE) void kq_gemv16_kernel(const KqArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+__device__ __forceinline__ void kq_body(const KqArgs& a, int bid, uint8_t* lds) {
   constexpr KGeo G = kgeo(F);
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(kWaves * TLX_WAVE) void kq_gemv16_kernel(const KqAr
   uint8_t* stg = lds + xbytes + (is_q6(F) ? 0 : (size_t)M * ng * 4) + wave * 16 * G.rs;
 
   const int T = (N + 15) >> 4;
-  const int t0 = (int)blockIdx.x * a.tw;
+  const int t0 = bid * a.tw;
   const int I = min(a.tw, T - t0) * nb;
   const int lo = kq_range(I, wave), hi = kq_range(I, wave + 1);
 
@@ -405,6 +406,147 @@ __global__ __launch_bounds__(kWaves * TLX_WAVE) void kq_gemv16_kernel(const KqAr
   }
 }
 
+template <int F>
+__global__ __launch_bounds__(kWaves * TLX_WAVE) void kq_gemv16_kernel(const KqArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  kq_body<F>(a, (int)blockIdx.x, lds);
+}
+
+// ------------------------------------------------------------------ q/k/v of three formats
+// A Q6_K q, an IQ3_XXS k and a Q4_K or IQ3_XXS v in one launch.  A launch of its own costs each
+// matrix its start, the staging of the activations and its drain: for a k or v of 1024 rows that is
+// nearly all of it (12288 + 1024 + 1024 rows, K = 5120, M = 4: k 6.5, v 8.3 and q 15.2 us).
+// Here every workgroup takes a range of tiles of one matrix, sized so that the ranges of the three
+// end together and all are resident at once (kq_mix_plan).  At M = 1 / 4 / 8 / 11 / 16 the three
+// matrices take 15.7 / 16.4 / 17.2 / 18.0 / 33.4 us (26.8 / 28.6 / 32.8 / 33.8 / 55.5 as launches of
+// their own; from M = 13 on two row groups read the weights twice).  57 MB in 15.7 us is 3.6 TB/s:
+// bound by the loads a CU keeps in flight (two items a wave) and the launch's ~4 us start and drain.
+// Held to 128 VGPRs, so that two workgroups fit a CU, it is slower at every M (17.1 .. 35.8 us).
+
+// IQ3_XXS rows (GGUF blocks or packed rows), the arithmetic and the block -> wave split of the
+// 8-wave IQ3_XXS GEMV (so the results are the same bits where that one runs 8 waves), the
+// activations from LDS.  LDS: [staged X][4096-entry grid table][7 partial tiles]
+__host__ __device__ inline size_t k_iq3_lds_bytes(int M, int K) {
+  return k_x_bytes(M, K) + 4096 * sizeof(u2_t) + (kWaves - 1) * kSlot;
+}
+
+struct KIq3Blk {
+  u4_t qs;
+  u2_t sw;
+  uint32_t d;
+};
+
+__device__ __forceinline__ void kq_iq3_body(const KqArgs& a, int bid, uint8_t* lds, const float* gridf,
+                                            bool raw) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int M = a.M, N = a.N, K = a.K, nb = K >> 8;
+  const int XS = K + 8;
+  _Float16* xs = reinterpret_cast<_Float16*>(lds);
+  u2_t* tbl = reinterpret_cast<u2_t*>(lds + k_x_bytes(M, K));
+  f4_t* red = reinterpret_cast<f4_t*>(lds + k_x_bytes(M, K) + 4096 * sizeof(u2_t));
+
+  const int T = (N + 15) >> 4;
+  const int t0 = bid * a.tw, t1 = min(t0 + a.tw, T);
+  const int col = lane & 15, kq = lane >> 4;
+  const uint32_t rowb = 98u * (uint32_t)nb;
+  const uint32_t qst = raw ? 98u : 64u, sst = raw ? 98u : 32u, dst = raw ? 98u : 2u;
+  // block b of the lane's row of tile t (tail tile: clamp the loads, mask the stores)
+  auto load = [&](KIq3Blk& r, int t, int b) {
+    const uint32_t roff = (uint32_t)min(16 * t + col, N - 1) * rowb;
+    r.qs = tlx_ldu<u4_t>(a.w + (roff + (raw ? 2u : 0u) + 16u * kq + qst * (uint32_t)b));
+    r.sw = tlx_ldu<u2_t>(a.w + (roff + (raw ? 66u : 64u * nb) + 8u * kq + sst * (uint32_t)b));
+    r.d = tlx_ldu<uint16_t>(a.w + (roff + (raw ? 0u : 96u * nb) + dst * (uint32_t)b));
+  };
+  // the wave's next (tile, block); stays on the last one at the end, whose loads then repeat
+  int nt = t0, nblk = min(wave, nb - 1);
+  auto advance = [&] {
+    if (nblk + kWaves < nb) nblk += kWaves;
+    else if (nt + 1 < t1) {
+      ++nt;
+      nblk = min(wave, nb - 1);
+    }
+  };
+  KIq3Blk cur;
+  load(cur, nt, nblk);
+  {
+    const int pr = (K + 511) >> 9;
+    for (int p = wave; p < M * pr; p += kWaves) {
+      const int m = p / pr, j = p - m * pr;
+      if (512 * j + 8 * lane < K)
+        __builtin_amdgcn_global_load_lds(
+            (const void*)(a.x + (size_t)m * K + 512 * j + 8 * lane),
+            (__attribute__((address_space(3))) void*)(xs + m * XS + 512 * j), 16, 0, 0);
+    }
+  }
+  tlx_iq3_table(tbl, gridf);
+  __syncthreads();
+  const _Float16* xa = xs + min(col, M - 1) * XS + 64 * kq;
+
+  for (int t = t0; t < t1; ++t) {
+    f4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int b = wave; b < nb; b += kWaves) {
+      KIq3Blk nxt;
+      advance();
+      load(nxt, nt, nblk);
+      const _Float16 ks0 = (_Float16)((float)(2u * (cur.sw.x >> 28) + 1u) * 0.25f);
+      const _Float16 ks1 = (_Float16)((float)(2u * (cur.sw.y >> 28) + 1u) * 0.25f);
+      f4_t D = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const h8_t X = *reinterpret_cast<const h8_t*>(xa + 256 * b + 8 * c);
+        const uint32_t qd = cur.qs[c >> 1];
+        const uint32_t qw = (c & 1) ? (qd >> 16) : (qd & 0xFFFFu);
+        const uint32_t sidx = ((c < 4 ? cur.sw.x : cur.sw.y) >> (7 * (c & 3))) & 0x7Fu;
+        const _Float16 k = c < 4 ? ks0 : ks1;
+        const h8_t B = tlx_iq3_chunk(tbl, qw, sidx) * h8_t{k, k, k, k, k, k, k, k};
+        D = __builtin_amdgcn_mfma_f32_16x16x32_f16(X, B, D, 0, 0, 0);
+      }
+      acc += tlx_h2f((uint16_t)cur.d) * D;
+      cur = nxt;
+    }
+    // fixed-order reduction over the waves
+    if (wave > 0) red[(wave - 1) * 64 + lane] = acc;
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) acc += red[(w - 1) * 64 + lane];
+      const int n = 16 * t + col;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int m = 4 * kq + j;
+        if (n < N && m < M) a.out[(size_t)m * N + n] = tlx_f2h_bits(acc[j]);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+struct KMixSeg {
+  const uint8_t* w;
+  uint16_t* out;
+  int n, tw, wg0;   // rows, tiles per workgroup, first workgroup
+};
+struct KMixArgs {
+  KMixSeg seg[3];   // q, k, v
+  const _Float16* x;
+  const float* gridf;
+  int M, K, raw, v4;   // raw: k (and an IQ3_XXS v) as GGUF blocks; v4: v is Q4_K
+};
+
+template <int QF>
+__global__ __launch_bounds__(kWaves * TLX_WAVE) void kq_mix_kernel(const KMixArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int bx = (int)blockIdx.x;
+  const int s = bx < a.seg[1].wg0 ? 0 : bx < a.seg[2].wg0 ? 1 : 2;
+  const KMixSeg& g = a.seg[s];
+  const KqArgs k{g.w, a.x, g.out, a.M, g.n, a.K, g.tw};
+  const int bid = bx - g.wg0;
+  if (s == 0) kq_body<QF>(k, bid, lds);
+  else if (s == 2 && a.v4) kq_body<KF_Q4K>(k, bid, lds);
+  else kq_iq3_body(k, bid, lds, a.gridf, a.raw != 0);
+}
+
 // largest row group whose staged activations fit the LDS budget
 inline int k_rows_per_pass(int F, int M, int K) {
   int mc = M;
@@ -445,10 +587,71 @@ int kq_gemv16_launch(const uint8_t* w, const _Float16* x, uint16_t* out, int M, 
   return TLX_OK;
 }
 
+template <int QF>
+hipError_t kq_mix_attr_once() {
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [] {
+    attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&kq_mix_kernel<QF>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
+  });
+  return attr;
+}
+
+inline size_t k_mix_lds_bytes(int QF, int M, int K, bool v4) {
+  return std::max({k_lds_bytes(QF, M, K), k_iq3_lds_bytes(M, K), v4 ? k_lds_bytes(KF_Q4K, M, K) : size_t(0)});
+}
+
+// Tiles per workgroup for the three matrices on `cus` workgroups, one a CU (VGPR-bound): the
+// smallest q range for which ranges of k and v of no more cost leave everything resident, then k
+// and v spread over the CUs that q leaves.  The cost of a tile is its bytes; an IQ3_XXS byte counts
+// twice (two table gathers per 4 weights' 1.5 bytes, where a nibble is a few packed instructions).
+void kq_mix_plan(const int64_t (&cost)[3], const int (&T)[3], int cus, int (&tw)[3]) {
+  auto wgs = [&](int i) { return (T[i] + tw[i] - 1) / tw[i]; };
+  for (int tq = std::max(1, T[0] / cus);; ++tq) {
+    for (int i = 0; i < 3; ++i) tw[i] = (int)std::min<int64_t>(T[i], std::max<int64_t>(1, tq * cost[0] / cost[i]));
+    const int g = wgs(0) + wgs(1) + wgs(2);
+    if (g <= std::max(cus, 3)) break;
+  }
+  const int most[3] = {tw[0], tw[1], tw[2]};
+  tw[1] = tw[2] = 1;
+  while (wgs(0) + wgs(1) + wgs(2) > std::max(cus, 3) && (tw[1] < most[1] || tw[2] < most[2])) {
+    const bool k = tw[2] >= most[2] || (tw[1] < most[1] && (tw[1] + 1) * cost[1] <= (tw[2] + 1) * cost[2]);
+    ++tw[k ? 1 : 2];
+  }
+}
+
+template <int QF>
+int kq_mix_launch(KMixArgs a, int M, int mc, hipStream_t st) {
+  const hipError_t attr = kq_mix_attr_once<QF>();
+  if (attr != hipSuccess) return (int)attr;
+  const int64_t cost[3] = {kgeo(QF).bs, 2 * 98, a.v4 ? kgeo(KF_Q4K).bs : 2 * 98};
+  int T[3], tw[3], grid = 0;
+  for (int i = 0; i < 3; ++i) T[i] = (a.seg[i].n + 15) / 16;
+  kq_mix_plan(cost, T, tlx_cu_count(), tw);
+  for (int i = 0; i < 3; ++i) {
+    a.seg[i].tw = tw[i];
+    a.seg[i].wg0 = grid;
+    grid += (T[i] + tw[i] - 1) / tw[i];
+  }
+  const _Float16* x = a.x;
+  uint16_t* const out[3] = {a.seg[0].out, a.seg[1].out, a.seg[2].out};
+  for (int m0 = 0; m0 < M; m0 += mc) {
+    a.M = std::min(mc, M - m0);
+    a.x = x + (size_t)m0 * a.K;
+    for (int i = 0; i < 3; ++i) a.seg[i].out = out[i] + (size_t)m0 * a.seg[i].n;
+    kq_mix_kernel<QF><<<grid, kWaves * TLX_WAVE, k_mix_lds_bytes(QF, a.M, a.K, a.v4 != 0), st>>>(a);
+    const int rc = tlx_launch_status();
+    if (rc != TLX_OK) return rc;
+  }
+  return TLX_OK;
+}
+
 }  // namespace
 
 int tlx_kq_setup() {
-  const hipError_t e[4] = {kq_attr_once<0>(), kq_attr_once<1>(), kq_attr_once<2>(), kq_attr_once<3>()};
+  const hipError_t e[6] = {kq_attr_once<0>(), kq_attr_once<1>(), kq_attr_once<2>(), kq_attr_once<3>(),
+                           kq_mix_attr_once<KF_Q6R>(), kq_mix_attr_once<KF_Q6P>()};
   for (hipError_t x : e)
     if (x != hipSuccess) return (int)x;
   return TLX_OK;
@@ -543,6 +746,27 @@ int tlx_kq_gemv(int fmt, const void* w, const uint16_t* x_f16, uint16_t* out_f16
   const int rc = kq_check(fmt, w, x_f16, out_f16, M, N, K);
   TLX_RET_IF(rc != TLX_OK || !launch, rc);
   return kq_gemv16(fmt, w, x_f16, out_f16, M, N, K, (hipStream_t)stream);
+}
+
+int tlx_kq_mix(int fmt, const void* const* w, uint16_t* const* out, const int* n, const float* gridf,
+               const uint16_t* x_f16, int M, int K, bool kraw, bool v4, bool* done, void* stream) {
+  TLX_RET_IF(!is_q6(fmt), TLX_E_ARG);
+  // One launch where it reads the q rows no more often than a launch of q alone does: the row group
+  // is the one whose activations fit beside each matrix's own LDS.  Where a larger K leaves the
+  // three together fewer rows, they keep a launch each.
+  int mc = M;
+  while (mc > 1 && k_mix_lds_bytes(fmt, mc, K, v4) > (size_t)kLdsMax) --mc;
+  *done = k_mix_lds_bytes(fmt, mc, K, v4) <= (size_t)kLdsMax && mc == k_rows_per_pass(fmt, M, K);
+  if (!*done) return TLX_OK;
+  KMixArgs a{};
+  for (int i = 0; i < 3; ++i) a.seg[i] = KMixSeg{(const uint8_t*)w[i], out[i], n[i], 0, 0};
+  a.x = (const _Float16*)x_f16;
+  a.gridf = gridf;
+  a.K = K;
+  a.raw = kraw;
+  a.v4 = v4;
+  return fmt == KF_Q6R ? kq_mix_launch<KF_Q6R>(a, M, mc, (hipStream_t)stream)
+                       : kq_mix_launch<KF_Q6P>(a, M, mc, (hipStream_t)stream);
 }
 
 extern "C" int tlx_q6k_gemv16(const void* w, const uint16_t* x_f16, uint16_t* out_f16, int M, int N,
