@@ -346,6 +346,10 @@ int tlx_moe_topk(const float* logits, uint16_t* eids, float* gates, int P, void*
  * Replaces rt8e256 (engine/mm/MM_P1_rt8e256.cu:14-21): rt8e256(wrt, wsh, h, eids, gates, sg). */
 int tlx_moe_route(const float* wrt, const float* wsh, const float* h, uint16_t* eids, float* gates,
                   float* sg, int P, void* stream);
+/* The same with the logits through caller-owned memory, f32[P][256], 16-B aligned (written): every
+ * router row on a workgroup of its own, then tlx_moe_topk.  The faster form up to about 96 positions. */
+int tlx_moe_route_logits(const float* wrt, const float* wsh, const float* h, float* logits, uint16_t* eids,
+                         float* gates, float* sg, int P, void* stream);
 
 /* Deterministic stable sort of the np = 8P pairs by expert (eids 8-B aligned): eoff i32[257] (exclusive bin
  * offsets), plist u16[np] (pair ids, pair order inside a bin), items u32[tlx_moe_max_items(np)]

@@ -141,9 +141,10 @@ def test_moe_route(gpu):
     np.testing.assert_allclose(sg.cpu().numpy(), ref_sg, rtol=1e-5)
 
 
-@pytest.mark.parametrize("P", [1, 3, 257, 1027])
+@pytest.mark.parametrize("P", [1, 3, 4, 5, 96, 97, 257, 1027])
 def test_moe_route_batches(gpu, P):
-    """Every positions-a-workgroup form (1, 4, 8) with a ragged last workgroup: logits in float64 decide
+    """A workgroup per router row (up to 96 positions; fewer than, as many as and more than its four
+    waves), and every positions-a-workgroup form (1, 4, 8) with a ragged last workgroup: logits in float64 decide
     the ids where the 8th and 9th are apart by more than fp32 sums of 2048 terms can move (1e-4)."""
     print(f"[case] moe route P={P}", flush=True)
     rng = np.random.default_rng(1200 + P)
@@ -185,7 +186,28 @@ def test_moe_topk_extremes(gpu):
     ref_e, ref_g = moe.topk_ref(lg)
     assert np.array_equal(eids.cpu().numpy().view(np.uint16), ref_e)
     np.testing.assert_allclose(gates.cpu().numpy(), ref_g, rtol=2e-6, atol=1e-7)
+    ops.moe_topk(torch.full((1, moe.E), float("nan"), device=gpu), eids[:1], gates[:1])
+    assert eids[0].tolist() == list(range(8)) and gates[0].isnan().all()   # eight different experts
 
+
+def test_moe_route_given_stream(gpu):
+    """A call with a stream of its own takes the form without the logits buffer, at any batch."""
+    print("[case] moe route on a given stream", flush=True)
+    rng = np.random.default_rng(1300)
+    wrt = torch.from_numpy((rng.standard_normal((moe.E, moe.HID)) * 0.02).astype(np.float32)).to(gpu)
+    wsh = torch.from_numpy((rng.standard_normal(moe.HID) * 0.02).astype(np.float32)).to(gpu)
+    h = torch.from_numpy(rng.standard_normal((5, moe.HID)).astype(np.float32)).to(gpu)
+    out = [(torch.empty(5, 8, dtype=torch.int16, device=gpu), torch.empty(5, 8, device=gpu), torch.empty(5, device=gpu))
+           for _ in range(2)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    ops.moe_route(wrt, wsh, h, *out[0])
+    ops.moe_route(wrt, wsh, h, *out[1], stream=side)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][0], out[1][0])
+    # fp32 sums of 2048 products in two orders
+    torch.testing.assert_close(out[0][1], out[1][1], rtol=1e-5, atol=0)
+    torch.testing.assert_close(out[0][2], out[1][2], rtol=1e-5, atol=0)
 
 
 @pytest.mark.parametrize("P", [11, 2048])

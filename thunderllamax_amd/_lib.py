@@ -79,6 +79,7 @@ SIGNATURES = {
     "tlx_p8w4_ffn": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p],
     "tlx_moe_topk": [_p, _p, _p, _i, _p],
     "tlx_moe_route": [_p, _p, _p, _p, _p, _p, _i, _p],
+    "tlx_moe_route_logits": [_p, _p, _p, _p, _p, _p, _p, _i, _p],
     "tlx_moe_sort": [_p, _p, _p, _p, _p, _i, _p],
     "tlx_moe_max_items": [_i],
     "tlx_moe_up4": [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _p],

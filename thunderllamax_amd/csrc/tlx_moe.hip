@@ -84,7 +84,7 @@ __device__ __forceinline__ void topk8_wave(float4 in, int lane, uint16_t* eids, 
     if (lane == r) { id = best; val = m; }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (4 * lane + j == best) v[j] = -3.402823466e38f;
+      if (any && 4 * lane + j == best) v[j] = -3.402823466e38f;
   }
   const float e = expf(val - first);
   float s8 = 0.f;
@@ -175,6 +175,55 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __re
 #pragma unroll
       for (int i = 0; i < kRtThreads / TLX_WAVE; ++i) s += shp[wave][i];
       sg[p] = 1.f / (1.f + expf(-s));
+    }
+  }
+}
+
+// The same logits with a workgroup per router row (row 256 is wsh, whose sums end as sg) and the
+// positions dealt to its four waves: a wave holds the row's 8 KB in 32 registers and reads each
+// position's h against it, two positions in flight.  wrt then comes through every CU's load path
+// instead of one CU's per position; the logits go through memory to moe_topk_kernel.  Both launches, us
+// at P = 1 / 4 / 16 / 64 / 128: 5.7 / 6.5 / 8.8 / 15.9 / 24.9 (1 wave 5.6 / 6.9 / 12.2 / 31 / 57, 8 waves
+// 5.5 / 6.4 / 9.2 / 15.3 / 23.5) against 21.2 / 23.1 / 23.5 / 22.7 / 22.7 of moe_route_kernel.  Bound by the two
+// launches at few positions, from 16 on by h, which every workgroup reads whole (8 KB a position and CU).
+constexpr int kLgWaves = 4;
+__global__ __launch_bounds__(kLgWaves * TLX_WAVE) void moe_logits_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
+                                                                         const float* __restrict__ h, float* __restrict__ logits,
+                                                                         float* __restrict__ sg, int P) {
+  const int row = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  constexpr int kPer = kHid / 4 / TLX_WAVE;
+  const float4* hp = reinterpret_cast<const float4*>(h) + lane;
+  float4 w[kPer], x[kPer];
+  if (wave >= P) return;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int k4 = TLX_WAVE * i + lane;
+    if (row < kE) {
+      w[i] = reinterpret_cast<const float4*>(wrt + (size_t)row * kHid)[k4];
+    } else {   // (wsh is 8-B aligned)
+      const float2 a = reinterpret_cast<const float2*>(wsh)[2 * k4], b = reinterpret_cast<const float2*>(wsh)[2 * k4 + 1];
+      w[i] = float4{a.x, a.y, b.x, b.y};
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) x[i] = hp[(size_t)wave * (kHid / 4) + TLX_WAVE * i];
+  for (int p = wave; p < P; p += kLgWaves) {
+    const float4* hn = hp + (size_t)min(p + kLgWaves, P - 1) * (kHid / 4);   // past the end: the last position again
+    float4 n[kPer], s = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) n[i] = hn[TLX_WAVE * i];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      s.x += w[i].x * x[i].x;
+      s.y += w[i].y * x[i].y;
+      s.z += w[i].z * x[i].z;
+      s.w += w[i].w * x[i].w;
+      x[i] = n[i];
+    }
+    const float v = wave_sum((s.x + s.y) + (s.z + s.w));
+    if (lane == 0) {
+      if (row < kE) logits[(size_t)p * kE + row] = v;
+      else sg[p] = 1.f / (1.f + expf(-v));
     }
   }
 }
@@ -1184,6 +1233,17 @@ extern "C" int tlx_moe_route(const float* wrt, const float* wsh, const float* h,
   if (P <= kRt1) return moe_route_launch<1>(wrt, wsh, h, eids, gates, sg, P, st);
   if (P <= kRt4) return moe_route_launch<4>(wrt, wsh, h, eids, gates, sg, P, st);
   return moe_route_launch<8>(wrt, wsh, h, eids, gates, sg, P, st);
+}
+
+extern "C" int tlx_moe_route_logits(const float* wrt, const float* wsh, const float* h, float* logits, uint16_t* eids,
+                                    float* gates, float* sg, int P, void* stream) {
+  TLX_RET_IF(P < 1, TLX_E_ARG);
+  TLX_RET_IF(!tlx_aligned(wrt, 16) || !tlx_aligned(h, 16) || !tlx_aligned(wsh, 8) || !tlx_aligned(logits, 16), TLX_E_ALIGN);
+  const hipStream_t st = (hipStream_t)stream;
+  moe_logits_kernel<<<kE + 1, kLgWaves * TLX_WAVE, 0, st>>>(wrt, wsh, h, logits, sg, P);
+  const int rc = tlx_launch_status();
+  TLX_RET_IF(rc != TLX_OK, rc);
+  return tlx_moe_topk(logits, eids, gates, P, stream);
 }
 
 extern "C" int tlx_moe_sort(const uint16_t* eids, int* eoff, uint16_t* plist, uint32_t* items, uint32_t* nitp,

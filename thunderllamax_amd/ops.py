@@ -631,6 +631,11 @@ def moe_topk(logits, eids, gates, stream=None):
     call("tlx_moe_topk", logits.data_ptr(), eids.data_ptr(), gates.data_ptr(), logits.shape[0], _stream(stream))
 
 
+# Largest batch the router takes with a workgroup per router row and the logits in memory: at 64
+# positions 15.9 us against 22.7 with whole positions a workgroup, at 128 24.9 against 22.7.
+MOE_ROUTE_LOGITS_MAX_P = 96
+
+
 def moe_route(wrt, wsh, h, eids, gates, sg, stream=None):
     """rt8e256(wrt, wsh, h, eids, gates, sg)."""
     P = h.shape[0]
@@ -641,6 +646,12 @@ def moe_route(wrt, wsh, h, eids, gates, sg, stream=None):
     _need(gates, P * 8 * 4, "gates")
     _need(sg, P * 4, "sg")
     _dev(wrt, wsh, h, eids, gates, sg)
+    # (the logits belong to the current stream; a call on another one takes the form without them)
+    if stream is None and 0 < P <= MOE_ROUTE_LOGITS_MAX_P:
+        logits = torch.empty(P, 256, dtype=torch.float32, device=h.device)
+        call("tlx_moe_route_logits", wrt.data_ptr(), wsh.data_ptr(), h.data_ptr(), logits.data_ptr(), eids.data_ptr(),
+             gates.data_ptr(), sg.data_ptr(), P, _stream(None))
+        return
     call("tlx_moe_route", wrt.data_ptr(), wsh.data_ptr(), h.data_ptr(), eids.data_ptr(), gates.data_ptr(),
          sg.data_ptr(), h.shape[0], _stream(stream))
 
