@@ -482,7 +482,7 @@ int tlx_moe_dn6(const uint64_t* ptbl_dn, const uint32_t* items, const uint32_t* 
 int tlx_moe_dn6_pairs(const uint64_t* ptbl_dn, const uint16_t* eids, const float* act, uint16_t* parts,
                       int np, int layout, void* stream);
 /* The sorted forms (tlx_moe_up3s / tlx_moe_dn6) and the Q8_0 shared expert's gate+up / down
- * (tlx_moe_shared8's two launches) in one launch each above P = 16 (else the two launches): the
+ * (tlx_moe_shared8's two launches) in one launch each above P = 512 (else the two launches): the
  * shared expert's workgroups follow the routed ones.  The down keeps two launches whenever parts
  * is 8-B aligned (the routed register-decode form and the shared expert's staged form have LDS
  * footprints one launch cannot share).  No counterpart in the reference (gxu_gm / gxm_dn6 and
@@ -495,7 +495,7 @@ int tlx_moe_dn6_sh(const uint64_t* ptbl_dn, const uint32_t* items, const uint32_
                    const uint16_t* plist, const float* act, uint16_t* parts, int np, const void* wd8,
                    const float* sact, float* shared, int P, int layout, void* stream);
 /* The pair walks (tlx_moe_up3s_pairs / tlx_moe_dn6_pairs) and the Q8_0 shared expert's decode forms
- * (tlx_moe_shared8's two launches) in one launch each at P <= 16 (else the two launches): the shared
+ * (tlx_moe_shared8's two launches) in one launch each at P <= 64 (else the two launches): the shared
  * expert's workgroups follow the pairs' and read their token rows from memory (no LDS staging, so
  * the pair walk keeps its occupancy).  No counterpart in the reference (gx8e256up / gx8e256dn6 and
  * shexp8 are separate launches); outputs those of the separate calls bit for bit.  sact f32 [P][512]
@@ -506,7 +506,7 @@ int tlx_moe_up3s_pairs_sh(const uint64_t* ptbl, const uint16_t* eids, const floa
 int tlx_moe_dn6_pairs_sh(const uint64_t* ptbl_dn, const uint16_t* eids, const float* act, uint16_t* parts, int np,
                          const void* wd8, const float* sact, float* shared, int P, int layout, void* stream);
 /* The Q8_0 shared expert over P positions: y[P][2048] f32 = Wd . (silu(Wg . x) * (Wu . x)), with act
- * f32[P][512] caller scratch (two launches on the stream; P <= 16 the decode form).  Replaces shexp8
+ * f32[P][512] caller scratch (two launches on the stream; P <= 512 the decode form).  Replaces shexp8
  * (engine/mm/MM_P2_shexp8.cu:8-13): shexp8(wg [512][2176], wu [512][2176], wd [2048][544], x, y).
  * x and act 16-B aligned. */
 int tlx_moe_shared8(const void* wg, const void* wu, const void* wd, const float* x, float* y, float* act, int P,

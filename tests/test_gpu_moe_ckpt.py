@@ -183,10 +183,10 @@ def test_ckpt_shared_q80(gpu, ckpt, P):
     assert _rows_err(y.cpu().numpy(), ref) <= TOL
 
 
-@pytest.mark.parametrize("P", [11, 300])
+@pytest.mark.parametrize("P", [11, 300, 520])
 def test_ckpt_grouped_shared_fused(gpu, ckpt, P):
     """moe_up3s_sh / moe_dn6_sh (the sorted forms and the Q8_0 shared expert in one launch each
-    above P = 16, two launches at P = 11) against moe_up3s / moe_dn6 / moe_shared8, bit for bit."""
+    above P = 512, two launches below) against moe_up3s / moe_dn6 / moe_shared8, bit for bit."""
     print(f"[case] sorted forms + Q8_0 shared expert in one launch, P={P}", flush=True)
     rng = np.random.default_rng(60 + P)
     x, eids, deids, eoff, plist, items, nitp = _route(gpu, rng, P)
@@ -210,6 +210,41 @@ def test_ckpt_grouped_shared_fused(gpu, ckpt, P):
         assert np.array_equal(a.view(v), b.view(v)), k
     ref = moe.shared8_ref(*ckpt["shared"], x)
     assert _rows_err(fus["shared"].cpu().numpy(), ref) <= TOL
+
+
+@pytest.mark.parametrize("P", [24, 512, 513])
+def test_ckpt_sorted_up_ragged(gpu, ckpt, ckpt_tiled, P):
+    """The sorted gate+up where experts hold 0, 1, 15, 16, 17 and more pairs (one pass of 16 tokens and
+    several), on both sides of the register-decode form's 4096 pairs, and the shared expert on both
+    sides of its 512 positions."""
+    print(f"[case] sorted gate+up, ragged experts, P={P}", flush=True)
+    rng = np.random.default_rng(70 + P)
+    x, eids, deids, eoff, plist, items, nitp = _route(gpu, rng, P)
+    cold = np.array([e for e in range(40, 256)])
+    eids = eids.reshape(P, 8).copy()
+    for p in range(P):
+        eids[p] = rng.choice(cold, 8, replace=False)
+        hot = [e for e, n in ((3, 1), (7, 15), (11, 16), (13, 17), (17, 24)) if p < n]
+        eids[p, :len(hot)] = hot
+    eids = eids.reshape(-1)
+    deids = torch.from_numpy(eids.view(np.int16)).to(gpu)
+    ops.moe_sort(deids, eoff, plist, items, nitp)
+    dx = torch.from_numpy(x).to(gpu)
+    acts = []
+    for pt, lay in ((ckpt["ptbl"], LAYOUT_RAW), (ckpt_tiled["ptbl"], LAYOUT_TILED)):
+        act = torch.full((8 * P + 1, moe.FF), -3.0, device=gpu)
+        ops.moe_up3s(pt, eoff, plist, dx, ckpt["gridf"], act[:8 * P], layout=lay)
+        acts.append(act.cpu().numpy())
+    assert np.array_equal(acts[0].view(np.uint32), acts[1].view(np.uint32))
+    assert (acts[0][8 * P] == -3.0).all()
+    for e in (3, 7, 11, 13, 17):
+        prs = np.nonzero(eids == e)[0]
+        ref = moe.up3s_ref(ckpt["gu"][e], ckpt["grid"], x[prs // 8])
+        assert _rows_err(acts[0][prs], ref) <= TOL, e
+    y, sact = torch.full((P + 1, moe.HID), -3.0, device=gpu), torch.empty(P, moe.FF, device=gpu)
+    ops.moe_shared8(*ckpt["dsh"], dx, y[:P], sact)
+    assert (y[P] == -3.0).all()
+    assert _rows_err(y[:P].cpu().numpy(), moe.shared8_ref(*ckpt["shared"], x)) <= TOL
 
 
 def test_ckpt_tiled_repack_matches_oracle(gpu, ckpt):
@@ -278,10 +313,11 @@ def test_ckpt_tiled_forms_bit_identical(gpu, ckpt, ckpt_tiled, P):
     _check_pairs(ckpt, x, eids, til["act"], til["parts"], list(range(0, np_, 7 if P <= 300 else 509)))
 
 
-@pytest.mark.parametrize("P,lay", [(1, LAYOUT_RAW), (11, LAYOUT_TILED), (16, LAYOUT_RAW), (17, LAYOUT_TILED)])
+@pytest.mark.parametrize("P,lay", [(1, LAYOUT_RAW), (11, LAYOUT_TILED), (16, LAYOUT_RAW), (17, LAYOUT_TILED),
+                                   (33, LAYOUT_RAW), (64, LAYOUT_TILED), (65, LAYOUT_RAW)])
 def test_ckpt_pairs_shared_fused(gpu, ckpt, ckpt_tiled, P, lay):
     """moe_up3s_pairs_sh / moe_dn6_pairs_sh (the pair walks and the Q8_0 shared expert in one launch
-    each at P <= 16, the two launches at P = 17) against moe_up3s_pairs / moe_dn6_pairs /
+    each up to P = 64, two launches at P = 65) against moe_up3s_pairs / moe_dn6_pairs /
     moe_shared8, bit for bit; the shared expert against the oracle."""
     print(f"[case] pair walks + Q8_0 shared expert in one launch, P={P} layout={lay}", flush=True)
     rng = np.random.default_rng(90 + P)

@@ -19,7 +19,7 @@
 // w runs v_mfma_f32_16x16x32_f16 over its 16 columns for every 16-token group of the pass.  Token
 // lists: sorted (the expert's bin from eoff / plist, in passes of 128) or dense (every position:
 // the shared expert).  gv_kernel (decode: the pair walk, one pair per item, pair p running expert
-// eids[p]; the shared expert at P <= 16): the same operands, built in registers (its section).
+// eids[p]; the shared expert up to 512 positions): the same operands, built in registers (its section).
 // gq_dn_kernel (the routed down over the sorted pairs): gv_kernel's register-built operands with
 // the expert's activations resident in LDS (its section).
 //
@@ -440,7 +440,8 @@ __global__ __launch_bounds__(64 * gx_waves<UP>()) void gx_kernel(const GxArgs a)
 // The sorted form (class RCLS) and the Q8_0 shared expert's dense form in one launch: workgroups
 // below nra run the routed experts (args a), the rest the shared expert (args b) -- each part its
 // own launch's code, so the outputs are the separate launches' bit for bit.  The shared expert's
-// workgroups come last, filling the routed grid's last round.
+// workgroups come last, filling the routed grid's last round (first: the same, layer at P = 1024 / 2048
+// 338 / 412 us against 334 / 414).
 template <int RCLS, bool UP, bool TL>
 __global__ __launch_bounds__(64 * gx_waves<UP>()) void gx_sh_kernel(const GxArgs a, const GxArgs b, int nra) {
   __shared__ GxLds<UP, RCLS == GX_IQ3S, gx_tok<GX_SORTED>()> L;   // the larger pass
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(64 * gx_waves<UP>()) void gx_sh_kernel(const GxArgs
 }
 
 // ------------------------------------------------------------------ decode form (GEMV-shaped)
-// Items of at most 16 tokens -- the pair walk (one token a pair) and the shared expert at P <= 16
+// Items of at most 16 tokens -- the pair walk (one token a pair) and the shared expert's positions
 // -- bypass the LDS weight stage: a 16-row tile (gate+up: the gate tile and its up tile) is walked
 // by KS waves, each over K / KS of k, in units of 256 weights.  Lane (col, kq) fetches the bytes
 // of row col that hold its 64 weights of a unit (contiguous in the record where the class allows)
@@ -587,7 +588,7 @@ struct GvShape {
   static constexpr int LDX = K + 8;                      // token row stride (halfs)
 };
 
-// XD (the dense form at P <= kGvTok): the token rows are read from memory (f32 -> fp16, as staged)
+// XD (the dense form beside a pair walk): the token rows are read from memory (f32 -> fp16, as staged)
 // a unit at a time instead of staged in LDS -- no LDS but the k-split sums, so the form can share a
 // launch with a pair walk (tlx_moe_up3s_pairs_sh) without lowering its occupancy; the same operands.
 template <int CLS, bool UP, int FORM, int KS, int NW, bool TL, bool XD>
@@ -741,7 +742,7 @@ __global__ __launch_bounds__(64 * NW) void gv_kernel(const GxArgs a) {
   gv_body<CLS, UP, FORM, KS, NW, TL, false>(xs, lslot, red, a, (int)blockIdx.x);
 }
 
-// The pair walk (class RCLS, 4 waves, KSR) and the Q8_0 shared expert's dense form at P <= kGvTok
+// The pair walk (class RCLS, 4 waves, KSR) and the Q8_0 shared expert's dense form
 // (direct token rows, 4 waves, KSS) in one launch: workgroups below nra walk the pairs (args a), the
 // rest run the shared expert (args b) -- each part its own code, the separate launches' bits.
 template <int RCLS, bool UP, int KSR, bool TL, int KSS>
@@ -768,6 +769,94 @@ int gv_launch(const GxArgs& a, int items, hipStream_t st) {
   const int nblk = FORM == GX_DENSE ? items * RB : (items + 7) / 8 * 8 * RB;
   gv_kernel<CLS, UP, FORM, KS, NW, TL><<<(unsigned)nblk, 64 * NW, 0, st>>>(b);
   return tlx_launch_status();
+}
+
+// The IQ3_S gate+up over the sorted pairs with register decode: an item is an expert, its tokens 16 at
+// a time staged as fp16 for the workgroup's TW tiles, the weights fetched and decoded again for each
+// 16 (gv_decode: the staged form's operands).  Where an expert has few tokens the staged form spends its
+// time on the chunk by chunk decode, barrier, MFMA chain of a workgroup; here the waves decode
+// independently.  Tiled slabs, P = 17 / 64 / 256 / 512: 52 / 83 / 101 / 141 us against the staged form's
+// 110 / 164 / 166 / 179 (bound by the decode's issue and its table reads).  Two units in flight and 128
+// VGPRs, so that two workgroups fit a CU: with all four units and 199 VGPRs 57 / 94 / 114 / 165 us, k over
+// four waves instead of two 60 / 105 / 135 / 197, fences between the steps of a unit 63 / 103 / 132 / 173.
+template <int KS, bool TL>
+__global__ __launch_bounds__(512, 4) void gvs_up_kernel(const GxArgs a) {
+  constexpr int NW = 8;
+  using S = GvShape<GX_IQ3S, true, GX_SORTED, KS, NW>;
+  constexpr int K = S::K, TW = S::TW, RB = S::RB, LDX = S::LDX, UW = S::NU / KS, DEPTH = 2;   // units in flight
+  constexpr int ROWB = K / GxFmt<GX_IQ3S>::kPer * GxFmt<GX_IQ3S>::kBlk;
+  static_assert(KS > 1, "the barrier of the k-split sums also frees the token rows for the next pass");
+  __shared__ __attribute__((aligned(16))) _Float16 xs[kGvTok * LDX];
+  __shared__ GvLutSlot<true> lslot;
+  __shared__ f4_t red[(KS - 1) * TW * 2 * 64];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, col = lane & 15, kq = lane >> 4;
+  const int tile = wave / KS, kp = wave % KS;
+  const int slot = (int)blockIdx.x >> 3, rb = slot % RB, e = slot / RB * 8 + ((int)blockIdx.x & 7);
+  if (e >= a.items) return;
+  const int end = a.eoff[e + 1];
+  int beg = a.eoff[e];
+  if (beg >= end) return;
+  gv_lut_fill<64 * NW>(lslot.v, a.grid, t);
+  const GvLut* lut = &lslot.v;
+  const int n = rb * (16 * TW) + 16 * tile + col;   // output column (weight row) of the lane
+  gbyte* const wg = reinterpret_cast<gbyte*>(a.ptbl[e]) + (size_t)n * ROWB;
+  gbyte* const rows[2] = {wg, wg + kIq3sGate};
+  const _Float16* xrow = xs + col * LDX;   // (rows past nt: not staged, their MFMA rows are not stored)
+  for (; beg < end; beg += kGvTok) {
+    const int nt = min(kGvTok, end - beg);
+    GvRaw<GX_IQ3S> raw[UW][2];
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) raw[u][m] = gv_fetch<GX_IQ3S, TL>(rows[m], kp * UW + u, kq);
+    int pair[4];   // the tokens 4 kq + r whose outputs the lane holds
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pair[r] = a.plist[min(beg + 4 * kq + r, end - 1)];
+    for (int pc = t; pc < nt * (K / 8); pc += 64 * NW) {
+      const int r = pc / (K / 8), k8 = pc - r * (K / 8);
+      const float4* src = reinterpret_cast<const float4*>(a.x + (size_t)(a.plist[beg + r] >> 3) * K + 8 * k8);
+      const float4 u = src[0], v = src[1];
+      *reinterpret_cast<h8_t*>(xs + r * LDX + 8 * k8) = h8_t{(_Float16)u.x, (_Float16)u.y, (_Float16)u.z, (_Float16)u.w,
+                                                             (_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+    }
+    __syncthreads();   // token rows, lookups
+    f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int u = 0; u < UW; ++u) {
+      if (u + DEPTH < UW) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m) raw[u + DEPTH][m] = gv_fetch<GX_IQ3S, TL>(rows[m], kp * UW + u + DEPTH, kq);
+      }
+      const _Float16* xu = xrow + 256 * (kp * UW + u);
+#define GVS_STEP(SS)                                                                 \
+  {                                                                                  \
+    const h8_t ax = *reinterpret_cast<const h8_t*>(xu + gv_koff<GX_IQ3S>(kq, SS));   \
+    _Pragma("unroll") for (int m = 0; m < 2; ++m) {                                  \
+      const h8_t bw = gv_decode<GX_IQ3S, SS>(raw[u][m], kq, lut);                    \
+      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax, bw, acc[m], 0, 0, 0);      \
+    }                                                                                \
+  }
+      GVS_STEP(0) GVS_STEP(1) GVS_STEP(2) GVS_STEP(3) GVS_STEP(4) GVS_STEP(5) GVS_STEP(6) GVS_STEP(7)
+#undef GVS_STEP
+    }
+    if (kp != 0) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) red[(((kp - 1) * TW + tile) * 2 + m) * 64 + lane] = acc[m];
+    }
+    __syncthreads();   // the sums; every wave is done with the token rows
+    if (kp == 0) {
+#pragma unroll
+      for (int j = 1; j < KS; ++j)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) acc[m] += red[(((j - 1) * TW + tile) * 2 + m) * 64 + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (4 * kq + r >= nt) continue;
+        const float gv = acc[0][r], uv = acc[1][r];
+        reinterpret_cast<float*>(a.out)[(size_t)pair[r] * kFf + n] = gv / (1.f + expf(-gv)) * uv;
+      }
+    }
+  }
 }
 
 // ------------------------------------------------------------------ batched down, register decode
@@ -1008,6 +1097,24 @@ extern "C" int tlx_q8_0_dequant(const void* w, void* out, int64_t rows, int64_t 
 // the slabs' layout argument: GGUF rows or this library's tiled records
 static bool ckpt_layout_ok(int layout) { return layout == TLX_LAYOUT_RAW || layout == TLX_LAYOUT_TILED; }
 
+// The register-decode form up to this many pairs (16 an expert on average: most experts then take one
+// pass): at 4096 pairs 141 us against 179, at 8192 268 against 195 (tiled slabs).
+constexpr int kGvsPairs = 4096, kGvsKs = 2;
+
+// the routed IQ3_S gate+up over the sorted pairs
+template <bool TL>
+static int up3s_sorted_tl(GxArgs a, int np, hipStream_t st) {
+  if (np > kGvsPairs) return gx_launch<GX_IQ3S, true, GX_SORTED, TL>(a, kE, st);
+  a.items = kE;
+  constexpr int RB = GvShape<GX_IQ3S, true, GX_SORTED, kGvsKs, 8>::RB;
+  gvs_up_kernel<kGvsKs, TL><<<(unsigned)((kE + 7) / 8 * 8 * RB), 512, 0, st>>>(a);
+  return tlx_launch_status();
+}
+
+static int up3s_sorted(const GxArgs& a, int np, int layout, hipStream_t st) {
+  return layout == TLX_LAYOUT_TILED ? up3s_sorted_tl<true>(a, np, st) : up3s_sorted_tl<false>(a, np, st);
+}
+
 extern "C" int tlx_moe_up3s(const uint64_t* ptbl, const int* eoff, const uint16_t* plist, const float* xs,
                             const float* gridf, float* ys, int np, int layout, void* stream) {
   TLX_RET_IF(!ptbl || !eoff || !plist || !xs || !gridf || !ys, TLX_E_ARG);
@@ -1015,8 +1122,7 @@ extern "C" int tlx_moe_up3s(const uint64_t* ptbl, const int* eoff, const uint16_
   TLX_RET_IF(!tlx_aligned(ptbl, 8) || !tlx_aligned(xs, 16) || !tlx_aligned(gridf, 16) || !tlx_aligned(ys, 4), TLX_E_ALIGN);
   GxArgs a{};
   a.ptbl = ptbl; a.eoff = eoff; a.plist = plist; a.x = xs; a.grid = gridf; a.out = ys;
-  if (layout == TLX_LAYOUT_TILED) return gx_launch<GX_IQ3S, true, GX_SORTED, true>(a, kE, (hipStream_t)stream);
-  return gx_launch<GX_IQ3S, true, GX_SORTED>(a, kE, (hipStream_t)stream);
+  return up3s_sorted(a, np, layout, (hipStream_t)stream);
 }
 
 extern "C" int tlx_moe_up3s_pairs(const uint64_t* ptbl, const uint16_t* eids, const float* xs, const float* gridf,
@@ -1072,35 +1178,40 @@ extern "C" int tlx_moe_dn6_pairs(const uint64_t* ptbl_dn, const uint16_t* eids, 
 
 // the shared expert's decode k-split (4 waves a workgroup: the shape the pair walks' launches share)
 constexpr int kShKsUp = 4, kShKsDn = 2;
+// Positions up to which it takes the decode form: both launches at P = 17 / 128 / 256 / 384 / 512 14.6 /
+// 15.4 / 22.8 / 40 / 46 us (the staged form 40 / 51 / 51 / 51 / 52, its few workgroups one chain of
+// chunks each), at 1024 87 against 53.  In the pair walks' launches up to kPshP, past every pair walk
+// that pays: layer at P = 17 77 -> 66 us, 32 119 -> 109.
+constexpr int kShGvP = 512, kPshP = 64;
 
-// the shared expert's two launches (decode form at P <= kGvTok)
+// the shared expert's two launches (decode form at P <= kShGvP, 16 positions an item)
 static int moe_shared8_up(const void* wg, const void* wu, const float* x, float* act, int P, hipStream_t st) {
   GxArgs a{};
   a.w0 = (const uint8_t*)wg; a.w1 = (const uint8_t*)wu; a.x = x; a.out = act; a.P = P;
-  if (P <= kGvTok) return gv_launch<GX_Q80, true, GX_DENSE, kShKsUp, 4>(a, 1, st);
+  if (P <= kShGvP) return gv_launch<GX_Q80, true, GX_DENSE, kShKsUp, 4>(a, (P + kGvTok - 1) / kGvTok, st);
   return gx_launch<GX_Q80, true, GX_DENSE>(a, (P + gx_tok<GX_DENSE>() - 1) / gx_tok<GX_DENSE>(), st);
 }
 
 static int moe_shared8_dn(const void* wd, const float* act, float* y, int P, hipStream_t st) {
   GxArgs b{};
   b.w0 = (const uint8_t*)wd; b.x = act; b.out = y; b.P = P;
-  if (P <= kGvTok) return gv_launch<GX_Q80, false, GX_DENSE, kShKsDn, 4>(b, 1, st);
+  if (P <= kShGvP) return gv_launch<GX_Q80, false, GX_DENSE, kShKsDn, 4>(b, (P + kGvTok - 1) / kGvTok, st);
   return gx_launch<GX_Q80, false, GX_DENSE>(b, (P + gx_tok<GX_DENSE>() - 1) / gx_tok<GX_DENSE>(), st);
 }
 
-// the pair walk (a, np items) + the shared expert's dense form with direct token rows (b, P <= kGvTok)
+// the pair walk (a, np items) + the shared expert's dense form with direct token rows (b)
 template <int RCLS, bool UP, int KSR, bool TL, int KSS>
 static int gv_psh_launch(const GxArgs& a, int np, const GxArgs& b, hipStream_t st) {
   GxArgs ra = a, sb = b;
   ra.items = np;
-  sb.items = 1;
+  sb.items = (b.P + kGvTok - 1) / kGvTok;
   const int nra = (np + 7) / 8 * 8 * GvShape<RCLS, UP, GX_PAIRS, KSR, 4>::RB;
-  const int nsb = GvShape<GX_Q80, UP, GX_DENSE, KSS, 4>::RB;
+  const int nsb = sb.items * GvShape<GX_Q80, UP, GX_DENSE, KSS, 4>::RB;
   gv_psh_kernel<RCLS, UP, KSR, TL, KSS><<<(unsigned)(nra + nsb), 256, 0, st>>>(ra, sb, nra);
   return tlx_launch_status();
 }
 
-// routed sorted form (a, kE items) + the shared expert's dense form (b) in one launch, P > kGvTok
+// routed sorted form (a, kE items) + the shared expert's dense form (b) in one launch, P > kShGvP
 template <int RCLS, bool UP, bool TL>
 static int gx_sh_launch(const GxArgs& a, const GxArgs& b, hipStream_t st) {
   constexpr int RB = (UP ? kFf : kHid) / (16 * gx_waves<UP>());
@@ -1123,9 +1234,8 @@ extern "C" int tlx_moe_up3s_sh(const uint64_t* ptbl, const int* eoff, const uint
   const hipStream_t st = (hipStream_t)stream;
   GxArgs a{};
   a.ptbl = ptbl; a.eoff = eoff; a.plist = plist; a.x = xs; a.grid = gridf; a.out = ys;
-  if (P <= kGvTok) {   // the shared expert's decode form is another kernel: two launches
-    const int rc = layout == TLX_LAYOUT_TILED ? gx_launch<GX_IQ3S, true, GX_SORTED, true>(a, kE, st)
-                                              : gx_launch<GX_IQ3S, true, GX_SORTED>(a, kE, st);
+  if (P <= kShGvP || np <= kGvsPairs) {   // a register-decode form is another kernel: two launches
+    const int rc = up3s_sorted(a, np, layout, st);
     TLX_RET_IF(rc != TLX_OK, rc);
     return moe_shared8_up(wg8, wu8, xs, sact, P, st);
   }
@@ -1147,7 +1257,7 @@ extern "C" int tlx_moe_dn6_sh(const uint64_t* ptbl_dn, const uint32_t* items, co
   const hipStream_t st = (hipStream_t)stream;
   GxArgs a{};
   a.ptbl = ptbl_dn; a.eoff = eoff; a.plist = plist; a.x = act; a.out = parts;
-  if (P <= kGvTok) {
+  if (P <= kShGvP) {
     const int rc = dn6_sorted(a, layout, st);
     TLX_RET_IF(rc != TLX_OK, rc);
     return moe_shared8_dn(wd8, sact, shared, P, st);
@@ -1172,7 +1282,7 @@ extern "C" int tlx_moe_shared8(const void* wg, const void* wu, const void* wd, c
   TLX_RET_IF(!tlx_aligned(wg, 2) || !tlx_aligned(wu, 2) || !tlx_aligned(wd, 2), TLX_E_ALIGN);
   TLX_RET_IF(!tlx_aligned(x, 16) || !tlx_aligned(act, 16) || !tlx_aligned(y, 4), TLX_E_ALIGN);
   hipStream_t st = (hipStream_t)stream;
-  const int r = moe_shared8_up(wg, wu, x, act, P, st);   // decode (P <= 16): the GEMV-shaped form
+  const int r = moe_shared8_up(wg, wu, x, act, P, st);   // (up to kShGvP positions the decode form)
   TLX_RET_IF(r != TLX_OK, r);
   return moe_shared8_dn(wd, act, y, P, st);
 }
@@ -1188,7 +1298,7 @@ extern "C" int tlx_moe_up3s_pairs_sh(const uint64_t* ptbl, const uint16_t* eids,
   const hipStream_t st = (hipStream_t)stream;
   GxArgs a{};
   a.ptbl = ptbl; a.eids = eids; a.x = xs; a.grid = gridf; a.out = ys;
-  if (P > kGvTok) {   // the shared expert's batch form is another kernel: two launches
+  if (P > kPshP) {   // two launches
     const int rc = layout == TLX_LAYOUT_TILED ? gv_launch<GX_IQ3S, true, GX_PAIRS, 4, 4, true>(a, np, st)
                                               : gv_launch<GX_IQ3S, true, GX_PAIRS, 4, 4>(a, np, st);
     TLX_RET_IF(rc != TLX_OK, rc);
@@ -1210,7 +1320,7 @@ extern "C" int tlx_moe_dn6_pairs_sh(const uint64_t* ptbl_dn, const uint16_t* eid
   const hipStream_t st = (hipStream_t)stream;
   GxArgs a{};
   a.ptbl = ptbl_dn; a.eids = eids; a.x = act; a.out = parts;
-  if (P > kGvTok) {
+  if (P > kPshP) {
     const int rc = layout == TLX_LAYOUT_TILED ? gv_launch<GX_Q6K, false, GX_PAIRS, 1, 4, true>(a, np, st)
                                               : gv_launch<GX_Q6K, false, GX_PAIRS, 1, 4>(a, np, st);
     TLX_RET_IF(rc != TLX_OK, rc);

@@ -884,7 +884,7 @@ def moe_dn6(ptbl_dn, items, nitp, eoff, plist, act, parts, stream=None, layout=L
 
 def moe_up3s_sh(ptbl, eoff, plist, xs, gridf, ys, wg8, wu8, sact, stream=None, layout=LAYOUT_RAW):
     """moe_up3s over the sorted pairs and the Q8_0 shared expert's gate+up (wg8 / wu8 rows, into
-    sact [P][512], P = xs.shape[0]) in one launch above P = 16 (else the two launches); outputs
+    sact [P][512], P = xs.shape[0]) in one launch above P = 512 (else the two launches); outputs
     those of moe_up3s and moe_shared8's gate+up bit for bit."""
     n = ys.shape[0]
     P = xs.shape[0]
@@ -904,7 +904,7 @@ def moe_up3s_sh(ptbl, eoff, plist, xs, gridf, ys, wg8, wu8, sact, stream=None, l
 
 def moe_dn6_sh(ptbl_dn, items, nitp, eoff, plist, act, parts, wd8, sact, shared, stream=None, layout=LAYOUT_RAW):
     """moe_dn6 over the sorted pairs and the Q8_0 shared expert's down projection (wd8 rows, sact
-    [P][512] into shared [P][2048] f32, P = sact.shape[0]) in one launch above P = 16 (else the
+    [P][512] into shared [P][2048] f32, P = sact.shape[0]) in one launch above P = 512 (else the
     two launches); outputs those of the separate calls bit for bit."""
     n = act.shape[0]
     P = sact.shape[0]
@@ -935,7 +935,7 @@ def moe_dn6_pairs(ptbl_dn, eids, act, parts, stream=None, layout=LAYOUT_RAW):
 
 def moe_up3s_pairs_sh(ptbl, eids, xs, gridf, ys, wg8, wu8, sact, stream=None, layout=LAYOUT_RAW):
     """moe_up3s_pairs and the Q8_0 shared expert's gate+up (wg8 / wu8 rows, into sact [P][512],
-    P = sact.shape[0]) in one launch at P <= 16 (else the two launches); outputs those of
+    P = sact.shape[0]) in one launch at P <= 64 (else the two launches); outputs those of
     moe_up3s_pairs and moe_shared8's gate+up bit for bit."""
     n = ys.shape[0]
     P = sact.shape[0]
@@ -954,7 +954,7 @@ def moe_up3s_pairs_sh(ptbl, eids, xs, gridf, ys, wg8, wu8, sact, stream=None, la
 
 def moe_dn6_pairs_sh(ptbl_dn, eids, act, parts, wd8, sact, shared, stream=None, layout=LAYOUT_RAW):
     """moe_dn6_pairs and the Q8_0 shared expert's down projection (wd8 rows, sact [P][512] into
-    shared [P][2048] f32) in one launch at P <= 16 (else the two launches); the separate calls' bits."""
+    shared [P][2048] f32) in one launch at P <= 64 (else the two launches); the separate calls' bits."""
     n = act.shape[0]
     P = sact.shape[0]
     _need(ptbl_dn, 256 * 8, "ptbl_dn")
@@ -1008,6 +1008,9 @@ _SIDE_STREAMS = {}
 # launch it skips costs more than the expert slabs that two pairs of the batch share and the
 # pair walk reads twice.
 MOE_PAIR_WALK_MAX_P = 16
+# The same for the checkpoint's classes with a Q6_K down: layer, pair walk against sorted forms, tiled
+# slabs P = 32 109 / 151 us, 40 131 / 156, 48 154 / 159; GGUF rows 32 151 / 167, 40 184 / 171.
+MOE_CKPT_PAIR_WALK_MAX_P = {LAYOUT_TILED: 40, LAYOUT_RAW: 32}
 
 
 def moe_layer(logits, sg, xs, hres, y, ptbl, ptbl_dn, ptbl_sh, iq4nl, scratch, stream=None, overlap_shared=None,
@@ -1080,7 +1083,7 @@ def moe_layer_ckpt(logits, sg, xs, hres, y, ptbl, ptbl_dn, shared8, gridf, scrat
     slabs, gate/up and down alike (pack_iq3s_tiled, pack_q6k_tiled / pack_iq4_tiled)."""
     sc = scratch
     if pair_walk is None:
-        pair_walk = xs.shape[0] <= MOE_PAIR_WALK_MAX_P
+        pair_walk = xs.shape[0] <= (MOE_CKPT_PAIR_WALK_MAX_P.get(layout, 0) if down == "q6k" else MOE_PAIR_WALK_MAX_P)
     if overlap_shared is None:
         overlap_shared = False
     cur = stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.current_stream()
