@@ -482,8 +482,8 @@ int tlx_moe_dn6(const uint64_t* ptbl_dn, const uint32_t* items, const uint32_t* 
 int tlx_moe_dn6_pairs(const uint64_t* ptbl_dn, const uint16_t* eids, const float* act, uint16_t* parts,
                       int np, int layout, void* stream);
 /* The sorted forms (tlx_moe_up3s / tlx_moe_dn6) and the Q8_0 shared expert's gate+up / down
- * (tlx_moe_shared8's two launches) in one launch each above P = 512 (else the two launches): the
- * shared expert's workgroups follow the routed ones.  The down keeps two launches whenever parts
+ * (tlx_moe_shared8's two launches) in one launch each above P = 512 (else, and for the gate+up
+ * up to 6144 pairs, the two launches): the shared expert's workgroups follow the routed ones.  The down keeps two launches whenever parts
  * is 8-B aligned (the routed register-decode form and the shared expert's staged form have LDS
  * footprints one launch cannot share).  No counterpart in the reference (gxu_gm / gxm_dn6 and
  * shexp8 are separate launches); outputs those of the separate calls bit for bit.

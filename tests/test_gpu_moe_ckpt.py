@@ -183,10 +183,11 @@ def test_ckpt_shared_q80(gpu, ckpt, P):
     assert _rows_err(y.cpu().numpy(), ref) <= TOL
 
 
-@pytest.mark.parametrize("P", [11, 300, 520])
+@pytest.mark.parametrize("P", [11, 300, 520, 769])
 def test_ckpt_grouped_shared_fused(gpu, ckpt, P):
     """moe_up3s_sh / moe_dn6_sh (the sorted forms and the Q8_0 shared expert in one launch each
-    above P = 512, two launches below) against moe_up3s / moe_dn6 / moe_shared8, bit for bit."""
+    above P = 512, the gate+up above 768, two launches below) against moe_up3s / moe_dn6 /
+    moe_shared8, bit for bit."""
     print(f"[case] sorted forms + Q8_0 shared expert in one launch, P={P}", flush=True)
     rng = np.random.default_rng(60 + P)
     x, eids, deids, eoff, plist, items, nitp = _route(gpu, rng, P)
@@ -212,10 +213,10 @@ def test_ckpt_grouped_shared_fused(gpu, ckpt, P):
     assert _rows_err(fus["shared"].cpu().numpy(), ref) <= TOL
 
 
-@pytest.mark.parametrize("P", [24, 512, 513])
+@pytest.mark.parametrize("P", [24, 512, 513, 769])
 def test_ckpt_sorted_up_ragged(gpu, ckpt, ckpt_tiled, P):
     """The sorted gate+up where experts hold 0, 1, 15, 16, 17 and more pairs (one pass of 16 tokens and
-    several), on both sides of the register-decode form's 4096 pairs, and the shared expert on both
+    several), on both sides of the register-decode form's 6144 pairs, and the shared expert on both
     sides of its 512 positions."""
     print(f"[case] sorted gate+up, ragged experts, P={P}", flush=True)
     rng = np.random.default_rng(70 + P)
@@ -245,6 +246,75 @@ def test_ckpt_sorted_up_ragged(gpu, ckpt, ckpt_tiled, P):
     ops.moe_shared8(*ckpt["dsh"], dx, y[:P], sact)
     assert (y[P] == -3.0).all()
     assert _rows_err(y[:P].cpu().numpy(), moe.shared8_ref(*ckpt["shared"], x)) <= TOL
+
+
+def _bins(gpu, eids):
+    """The sorted bins of given expert ids."""
+    np_ = len(eids)
+    deids = torch.from_numpy(np.ascontiguousarray(eids, dtype=np.uint16).view(np.int16)).to(gpu)
+    eoff = torch.empty(257, dtype=torch.int32, device=gpu)
+    plist = torch.empty(np_, dtype=torch.int16, device=gpu)
+    items = torch.empty(ops.moe_max_items(np_), dtype=torch.int32, device=gpu)
+    ops.moe_sort(deids, eoff, plist, items, torch.empty(1, dtype=torch.int32, device=gpu))
+    return eoff, plist
+
+
+@pytest.mark.parametrize("counts", [
+    {255: 320},                                          # one expert, the last
+    {0: 512, 1: 33, 2: 32, 3: 17, 130: 16, 254: 1, 255: 29},   # neighbours in one lane's four experts
+    {8 * i + 3: 512 for i in range(8)},                  # 4096 pairs on 8 experts of one lane position
+    {5: 6144},                                           # the register-decode form's most, on one expert
+])
+def test_ckpt_sorted_up_concentrated(gpu, ckpt, ckpt_tiled, counts):
+    """The sorted gate+up where a few experts hold the pairs (many 16-token items an expert): every
+    pair written, nothing past them, sampled rows against the oracle, both layouts the same bits."""
+    print(f"[case] sorted gate+up, pairs a expert {counts}", flush=True)
+    rng = np.random.default_rng(sum(counts) + len(counts))
+    eids = rng.permutation(np.concatenate([np.full(n, e) for e, n in counts.items()]))
+    np_ = len(eids)
+    x = synth.bf16_round(0.05 * rng.standard_normal(((np_ + 7) // 8, moe.HID)).astype(np.float32))
+    eoff, plist = _bins(gpu, eids)
+    acts = []
+    for pt, lay in ((ckpt["ptbl"], LAYOUT_RAW), (ckpt_tiled["ptbl"], LAYOUT_TILED)):
+        act = torch.full((np_ + 1, moe.FF), float("nan"), device=gpu)
+        ops.moe_up3s(pt, eoff, plist, torch.from_numpy(x).to(gpu), ckpt["gridf"], act[:np_], layout=lay)
+        acts.append(act.cpu().numpy())
+    assert np.isfinite(acts[0][:np_]).all() and np.isnan(acts[0][np_]).all()
+    assert np.array_equal(acts[0].view(np.uint32), acts[1].view(np.uint32))
+    for e, n in counts.items():
+        prs = np.nonzero(eids == e)[0]
+        prs = prs[sorted({0, 15, 16, 31, 32, n // 2, n - 17, n - 16, n - 1} & set(range(n)))]   # ends of items
+        ref = moe.up3s_ref(ckpt["gu"][e], ckpt["grid"], x[prs // 8])
+        assert _rows_err(acts[0][prs], ref) <= TOL, e
+
+
+def test_ckpt_sorted_up_time_by_concentration(gpu, ckpt, ckpt_tiled):
+    """The sorted gate+up's time is that of its 16-token items, not of the expert that holds most: 4096
+    pairs on 8 experts (256 items) take no longer than spread over all (256 to 512 items), with a margin
+    of 2 for the clock (measured 0.9; 4.7 with a workgroup for all of an expert's items)."""
+    print("[case] sorted gate+up time, 4096 pairs on 8 experts against 256", flush=True)
+    P = 512
+    rng = np.random.default_rng(3)
+    dx = torch.from_numpy(synth.bf16_round(0.05 * rng.standard_normal((P, moe.HID)).astype(np.float32))).to(gpu)
+    act = torch.empty(8 * P, moe.FF, device=gpu)
+
+    def best(eids):
+        eoff, plist = _bins(gpu, eids)
+        ts = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(4):
+                ops.moe_up3s(ckpt_tiled["ptbl"], eoff, plist, dx, ckpt["gridf"], act, layout=LAYOUT_TILED)
+            b.record()
+            torch.cuda.synchronize()
+            ts.append(a.elapsed_time(b))
+        return min(ts)
+
+    spread = best(np.concatenate([rng.permutation(256)[:8] for _ in range(P)]))
+    hot = best(np.tile(np.arange(8) * 32 + 8, P))
+    print(f"[case] {spread / 4 * 1e3:.1f} us spread, {hot / 4 * 1e3:.1f} us on 8 experts", flush=True)
+    assert hot <= 2.0 * spread
 
 
 def test_ckpt_tiled_repack_matches_oracle(gpu, ckpt):

@@ -771,90 +771,124 @@ int gv_launch(const GxArgs& a, int items, hipStream_t st) {
   return tlx_launch_status();
 }
 
-// The IQ3_S gate+up over the sorted pairs with register decode: an item is an expert, its tokens 16 at
-// a time staged as fp16 for the workgroup's TW tiles, the weights fetched and decoded again for each
-// 16 (gv_decode: the staged form's operands).  Where an expert has few tokens the staged form spends its
+// The IQ3_S gate+up over the sorted pairs with register decode: an item is up to 16 of an expert's
+// tokens (one MFMA row tile), staged as fp16 for the workgroup's TW tiles; every item fetches and decodes
+// the expert's weights for itself (gv_decode: the staged form's operands), so no workgroup's time
+// depends on how many tokens its expert holds.
+// The items: the first kGvTok tokens of every expert, then the rest of the experts that hold more, found
+// from the bins in expert order (gvs_rest).  Where an expert has few tokens the staged form spends its
 // time on the chunk by chunk decode, barrier, MFMA chain of a workgroup; here the waves decode
-// independently.  Tiled slabs, P = 17 / 64 / 256 / 512: 52 / 83 / 101 / 141 us against the staged form's
-// 110 / 164 / 166 / 179 (bound by the decode's issue and its table reads).  Two units in flight and 128
-// VGPRs, so that two workgroups fit a CU: with all four units and 199 VGPRs 57 / 94 / 114 / 165 us, k over
-// four waves instead of two 60 / 105 / 135 / 197, fences between the steps of a unit 63 / 103 / 132 / 173.
+// independently.  us, tiled slabs, P = 17 / 64 / 256 / 512, uniform routing: 44 / 64 / 76 / 110 against the
+// staged form's 110 / 164 / 166 / 179; all positions on the same 8 experts, 64 / 256 / 512: 34 / 61 / 96
+// against 65 / 158 / 302.  (A workgroup walking all of its expert's tokens, 16 at a time: 57 / 85 / 102 / 148
+// and 93 / 353 / 694: the hottest expert was the launch; 32 tokens a workgroup 55 / 83 / 103 / 148 and 72 /
+// 92 / 134.)  Two units in flight and 128 VGPRs, so that two workgroups fit a CU: with all four units 45 /
+// 64 / 81 / 111, k over four waves instead of two 69 / 104 / 143 / 208.
+
+// item i of the tokens past every expert's first kGvTok: its expert and first pair, or false past the
+// last one (uniform over the wave; lane l looks at experts 4 l .. 4 l + 3)
+__device__ __forceinline__ bool gvs_rest(const int* eoff, int i, int& e, int& beg) {
+  const int lane = threadIdx.x & 63;
+  int off[5], n[4], sum = 0;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) off[q] = eoff[4 * lane + q];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    n[q] = (max(off[q + 1] - off[q], 1) - 1) / kGvTok;
+    sum += n[q];
+  }
+  int last = sum;   // items up to and with this lane's
+#pragma unroll
+  for (int d = 1; d < TLX_WAVE; d <<= 1) {
+    const int v = __shfl_up(last, d, TLX_WAVE);
+    if (lane >= d) last += v;
+  }
+  const uint64_t past = __ballot(last > i);
+  if (past == 0) return false;
+  int k = i - (last - sum), q = 0;
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    if (q == j && k >= n[j]) { k -= n[j]; ++q; }
+  const int first = (q == 0 ? off[0] : q == 1 ? off[1] : q == 2 ? off[2] : off[3]) + kGvTok * (k + 1);
+  const int at = __builtin_ctzll(past);   // the lane whose experts hold it
+  e = __builtin_amdgcn_readlane(4 * lane + q, at);
+  beg = __builtin_amdgcn_readlane(first, at);
+  return true;
+}
+
 template <int KS, bool TL>
 __global__ __launch_bounds__(512, 4) void gvs_up_kernel(const GxArgs a) {
   constexpr int NW = 8;
   using S = GvShape<GX_IQ3S, true, GX_SORTED, KS, NW>;
   constexpr int K = S::K, TW = S::TW, RB = S::RB, LDX = S::LDX, UW = S::NU / KS, DEPTH = 2;   // units in flight
   constexpr int ROWB = K / GxFmt<GX_IQ3S>::kPer * GxFmt<GX_IQ3S>::kBlk;
-  static_assert(KS > 1, "the barrier of the k-split sums also frees the token rows for the next pass");
   __shared__ __attribute__((aligned(16))) _Float16 xs[kGvTok * LDX];
   __shared__ GvLutSlot<true> lslot;
   __shared__ f4_t red[(KS - 1) * TW * 2 * 64];
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, col = lane & 15, kq = lane >> 4;
   const int tile = wave / KS, kp = wave % KS;
-  const int slot = (int)blockIdx.x >> 3, rb = slot % RB, e = slot / RB * 8 + ((int)blockIdx.x & 7);
-  if (e >= a.items) return;
-  const int end = a.eoff[e + 1];
-  int beg = a.eoff[e];
-  if (beg >= end) return;
+  const int slot = (int)blockIdx.x >> 3, rb = slot % RB, item = slot / RB * 8 + ((int)blockIdx.x & 7);
+  int e = item, beg;
+  if (item < kE) beg = a.eoff[e];
+  else if (!gvs_rest(a.eoff, item - kE, e, beg)) return;
+  const int nt = min(a.eoff[e + 1] - beg, kGvTok);
+  if (nt <= 0) return;
   gv_lut_fill<64 * NW>(lslot.v, a.grid, t);
   const GvLut* lut = &lslot.v;
   const int n = rb * (16 * TW) + 16 * tile + col;   // output column (weight row) of the lane
   gbyte* const wg = reinterpret_cast<gbyte*>(a.ptbl[e]) + (size_t)n * ROWB;
   gbyte* const rows[2] = {wg, wg + kIq3sGate};
   const _Float16* xrow = xs + col * LDX;   // (rows past nt: not staged, their MFMA rows are not stored)
-  for (; beg < end; beg += kGvTok) {
-    const int nt = min(kGvTok, end - beg);
-    GvRaw<GX_IQ3S> raw[UW][2];
+  GvRaw<GX_IQ3S> raw[UW][2];
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u)
+  for (int u = 0; u < DEPTH; ++u)
 #pragma unroll
-      for (int m = 0; m < 2; ++m) raw[u][m] = gv_fetch<GX_IQ3S, TL>(rows[m], kp * UW + u, kq);
-    int pair[4];   // the tokens 4 kq + r whose outputs the lane holds
+    for (int m = 0; m < 2; ++m) raw[u][m] = gv_fetch<GX_IQ3S, TL>(rows[m], kp * UW + u, kq);
+  int pair[4];   // the tokens 4 kq + r whose outputs the lane holds
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pair[r] = a.plist[min(beg + 4 * kq + r, end - 1)];
-    for (int pc = t; pc < nt * (K / 8); pc += 64 * NW) {
-      const int r = pc / (K / 8), k8 = pc - r * (K / 8);
-      const float4* src = reinterpret_cast<const float4*>(a.x + (size_t)(a.plist[beg + r] >> 3) * K + 8 * k8);
-      const float4 u = src[0], v = src[1];
-      *reinterpret_cast<h8_t*>(xs + r * LDX + 8 * k8) = h8_t{(_Float16)u.x, (_Float16)u.y, (_Float16)u.z, (_Float16)u.w,
-                                                             (_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
-    }
-    __syncthreads();   // token rows, lookups
-    f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int u = 0; u < UW; ++u) {
-      if (u + DEPTH < UW) {
-#pragma unroll
-        for (int m = 0; m < 2; ++m) raw[u + DEPTH][m] = gv_fetch<GX_IQ3S, TL>(rows[m], kp * UW + u + DEPTH, kq);
-      }
-      const _Float16* xu = xrow + 256 * (kp * UW + u);
-#define GVS_STEP(SS)                                                                 \
-  {                                                                                  \
-    const h8_t ax = *reinterpret_cast<const h8_t*>(xu + gv_koff<GX_IQ3S>(kq, SS));   \
-    _Pragma("unroll") for (int m = 0; m < 2; ++m) {                                  \
-      const h8_t bw = gv_decode<GX_IQ3S, SS>(raw[u][m], kq, lut);                    \
-      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax, bw, acc[m], 0, 0, 0);      \
-    }                                                                                \
+  for (int r = 0; r < 4; ++r) pair[r] = a.plist[min(beg + 4 * kq + r, beg + nt - 1)];
+  for (int pc = t; pc < nt * (K / 8); pc += 64 * NW) {
+    const int r = pc / (K / 8), k8 = pc - r * (K / 8);
+    const float4* src = reinterpret_cast<const float4*>(a.x + (size_t)(a.plist[beg + r] >> 3) * K + 8 * k8);
+    const float4 u = src[0], v = src[1];
+    *reinterpret_cast<h8_t*>(xs + r * LDX + 8 * k8) = h8_t{(_Float16)u.x, (_Float16)u.y, (_Float16)u.z, (_Float16)u.w,
+                                                           (_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
   }
-      GVS_STEP(0) GVS_STEP(1) GVS_STEP(2) GVS_STEP(3) GVS_STEP(4) GVS_STEP(5) GVS_STEP(6) GVS_STEP(7)
+  __syncthreads();   // token rows, lookups
+  f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int u = 0; u < UW; ++u) {
+    if (u + DEPTH < UW) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) raw[u + DEPTH][m] = gv_fetch<GX_IQ3S, TL>(rows[m], kp * UW + u + DEPTH, kq);
+    }
+    const _Float16* xu = xrow + 256 * (kp * UW + u);
+#define GVS_STEP(SS)                                                               \
+  {                                                                                \
+    const h8_t ax = *reinterpret_cast<const h8_t*>(xu + gv_koff<GX_IQ3S>(kq, SS)); \
+    _Pragma("unroll") for (int m = 0; m < 2; ++m) {                                \
+      const h8_t bw = gv_decode<GX_IQ3S, SS>(raw[u][m], kq, lut);                  \
+      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax, bw, acc[m], 0, 0, 0);    \
+    }                                                                              \
+  }
+    GVS_STEP(0) GVS_STEP(1) GVS_STEP(2) GVS_STEP(3) GVS_STEP(4) GVS_STEP(5) GVS_STEP(6) GVS_STEP(7)
 #undef GVS_STEP
-    }
-    if (kp != 0) {
+  }
+  if (kp != 0) {
 #pragma unroll
-      for (int m = 0; m < 2; ++m) red[(((kp - 1) * TW + tile) * 2 + m) * 64 + lane] = acc[m];
-    }
-    __syncthreads();   // the sums; every wave is done with the token rows
-    if (kp == 0) {
+    for (int m = 0; m < 2; ++m) red[(((kp - 1) * TW + tile) * 2 + m) * 64 + lane] = acc[m];
+  }
+  __syncthreads();   // the sums
+  if (kp == 0) {
 #pragma unroll
-      for (int j = 1; j < KS; ++j)
+    for (int j = 1; j < KS; ++j)
 #pragma unroll
-        for (int m = 0; m < 2; ++m) acc[m] += red[(((j - 1) * TW + tile) * 2 + m) * 64 + lane];
+      for (int m = 0; m < 2; ++m) acc[m] += red[(((j - 1) * TW + tile) * 2 + m) * 64 + lane];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (4 * kq + r >= nt) continue;
-        const float gv = acc[0][r], uv = acc[1][r];
-        reinterpret_cast<float*>(a.out)[(size_t)pair[r] * kFf + n] = gv / (1.f + expf(-gv)) * uv;
-      }
+    for (int r = 0; r < 4; ++r) {
+      if (4 * kq + r >= nt) continue;
+      const float gv = acc[0][r], uv = acc[1][r];
+      reinterpret_cast<float*>(a.out)[(size_t)pair[r] * kFf + n] = gv / (1.f + expf(-gv)) * uv;
     }
   }
 }
@@ -1097,17 +1131,19 @@ extern "C" int tlx_q8_0_dequant(const void* w, void* out, int64_t rows, int64_t 
 // the slabs' layout argument: GGUF rows or this library's tiled records
 static bool ckpt_layout_ok(int layout) { return layout == TLX_LAYOUT_RAW || layout == TLX_LAYOUT_TILED; }
 
-// The register-decode form up to this many pairs (16 an expert on average: most experts then take one
-// pass): at 4096 pairs 141 us against 179, at 8192 268 against 195 (tiled slabs).
-constexpr int kGvsPairs = 4096, kGvsKs = 2;
+// The register-decode form up to this many pairs (24 an expert on average), where the layer is faster
+// with it at every routing: layer, us, register decode / staged, uniform routing at 4608 / 6144 / 8192 pairs
+// tiled 255 / 308, 294 / 323, 338 / 335, GGUF rows 317 / 354, 368 / 374, 428 / 390; half the pairs on 8
+// experts tiled 411 / 659, 497 / 775, 630 / 953.
+constexpr int kGvsPairs = 6144, kGvsKs = 2;
 
 // the routed IQ3_S gate+up over the sorted pairs
 template <bool TL>
 static int up3s_sorted_tl(GxArgs a, int np, hipStream_t st) {
   if (np > kGvsPairs) return gx_launch<GX_IQ3S, true, GX_SORTED, TL>(a, kE, st);
-  a.items = kE;
   constexpr int RB = GvShape<GX_IQ3S, true, GX_SORTED, kGvsKs, 8>::RB;
-  gvs_up_kernel<kGvsKs, TL><<<(unsigned)((kE + 7) / 8 * 8 * RB), 512, 0, st>>>(a);
+  const int items = kE + (np - 1) / kGvTok;   // (an expert's items past its first: (its pairs - 1) / kGvTok)
+  gvs_up_kernel<kGvsKs, TL><<<(unsigned)((items + 7) / 8 * 8 * RB), 512, 0, st>>>(a);
   return tlx_launch_status();
 }
 

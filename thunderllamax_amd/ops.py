@@ -884,7 +884,7 @@ def moe_dn6(ptbl_dn, items, nitp, eoff, plist, act, parts, stream=None, layout=L
 
 def moe_up3s_sh(ptbl, eoff, plist, xs, gridf, ys, wg8, wu8, sact, stream=None, layout=LAYOUT_RAW):
     """moe_up3s over the sorted pairs and the Q8_0 shared expert's gate+up (wg8 / wu8 rows, into
-    sact [P][512], P = xs.shape[0]) in one launch above P = 512 (else the two launches); outputs
+    sact [P][512], P = xs.shape[0]) in one launch above P = 512 and 6144 pairs (else the two launches); outputs
     those of moe_up3s and moe_shared8's gate+up bit for bit."""
     n = ys.shape[0]
     P = xs.shape[0]
