@@ -159,34 +159,58 @@ def _units(gpu, seed, rows, kdim):
     return ops.pack_w7(w, torch.empty(rows * kdim // 2, dtype=torch.uint8, device=gpu), rows, kdim)
 
 
-@pytest.mark.parametrize("M,N,K,mib", [
-    (256, 5120, 17408, 128),    # 20 tiles: ranges that divide a tile (12 each)
-    (256, 5120, 17408, 11),     # the same with room for 44 parts: one range fewer or none
-    (512, 256, 4096, 128),      # 2 tiles of 32 chunks, at least 4 chunks a range
-    (2048, 5120, 2304, 128),    # 160 tiles of 18 chunks in 256 ranges: two segments a workgroup
-    (256, 17408 * 2, 5120, 128),   # 136 tiles of 40 chunks: two segments a workgroup
+def _parts_written(ws, mark):
+    """256 KB slots of the workspace that no longer hold the mark."""
+    return int((ws.view(torch.int32)[:ws.numel() // 4].view(-1, 1 << 16) != mark).any(dim=1).sum())
+
+
+# On 256 compute units: r tiles of K / 128 chunks; `parts` is G where G ranges divide the tiles, else
+# G + r - gcd(G, r) (one a range and tile).
+@pytest.mark.parametrize("M,N,K,mib,parts", [
+    (256, 5120, 17408, 128, 240),   # 20 tiles: ranges that divide a tile, 12 each
+    (256, 5120, 17408, 60, 240),    # the same in just 240 slots
+    (256, 5120, 17408, 20, 80),     # 80 slots: 4 each
+    (256, 5120, 17408, 11, 40),     # 44 slots: 2 each
+    (256, 5120, 17408, 8, 0),       # 32 slots: whole tiles
+    (512, 256, 4096, 128, 16),      # 2 tiles of 32 chunks, at least 4 chunks a range
+    (2048, 5120, 17408, 128, 384),  # 160 tiles in 256 ranges: two segments a workgroup
+    (2048, 5120, 17408, 104, 384),  # the same in the 415 slots that it asks for
+    (2048, 5120, 17408, 103, 0),    # one MiB less: whole tiles
+    (2048, 5120, 2304, 128, 0),     # 160 tiles of 18 chunks: whole tiles cost less than a split
+    (256, 17408 * 2, 5120, 128, 384),   # 136 tiles of 40 chunks: two segments a workgroup
+    (2048, 2048, 17408, 64, 256),   # 64 tiles in 256 slots: 4 ranges a tile
 ])
-def test_pfg3_split_ranges(gpu, M, N, K, mib):
-    """The split schedules against whole tiles (no workspace): the same products in another fp32 order
-    (at most K roundings of 2^-24 of the row's norm-wise sum: 1e-5 holds), every output written, and the
-    same bits on every call."""
+def test_pfg3_split_ranges(gpu, M, N, K, mib, parts):
+    """The split schedules against whole tiles (no workspace): the parts that the workspace's room
+    allows, the same products in another fp32 order (at most K roundings of 2^-24 of the row's norm-wise
+    sum: 1e-5 holds), every output written, and the same bits on every call."""
     print(f"[case] pfg3 split M={M} N={N} K={K} workspace {mib} MiB", flush=True)
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the parts are those of 256 compute units")
     grid = formats.gridf_tensor(gpu)
     g = torch.Generator(device=gpu)
     g.manual_seed(M + N + K)
     x = torch.randn(M, K, device=gpu, generator=g).half()
     res = torch.randn(M, N, device=gpu, generator=g)
     w = _units(gpu, 1, N, K)
+    mark = 0x7FABCDEF
     outs = []
     try:
         for size in (0, mib << 20, mib << 20):
-            ops.attach_workspace(gpu, gemm_bytes=size)
+            _, ws = ops.attach_workspace(gpu, gemm_bytes=size)
             y = torch.full((M, N), float("nan"), device=gpu)
-            ops.pfg3_iq3d(w, grid, x, res, y)
             ffn = torch.full((M, N // 2), float("nan"), dtype=torch.float16, device=gpu)
-            ops.pfg3_ffn(w[:w.numel() // 2], w[w.numel() // 2:], grid, x, ffn)
-            torch.cuda.synchronize()
+            written = []
+            for call_ in (lambda: ops.pfg3_iq3d(w, grid, x, res, y),
+                          lambda: ops.pfg3_ffn(w[:w.numel() // 2], w[w.numel() // 2:], grid, x, ffn)):
+                if ws is not None:
+                    ws.view(torch.int32).fill_(mark)
+                call_()
+                torch.cuda.synchronize()
+                if ws is not None:
+                    written.append(_parts_written(ws, mark))
             outs.append((y, ffn))
+            assert written == ([parts, parts] if size else []), written
     finally:
         ops.attach_workspace(gpu)
     (whole, fw), (split, fs), (again, fa) = outs

@@ -404,16 +404,23 @@ __device__ __forceinline__ void pf_kq_step(PfLds& L, f4_t (&acc)[kMI][8], const 
 // Schedule: `full` workgroups own one whole tile each (the complete rounds of one workgroup per
 // CU); the k-chunks of the remaining r tiles, tile after tile, are cut into G equal ranges, one per
 // workgroup of the last round.  A range is no longer than a tile (G > r), so it touches at most two:
-// its workgroup computes them one after the other as segments and stores each one's fp32 part in
-// slot 2 g or 2 g + 1; pf_fix_kernel sums a tile's parts in range order.  (Combining inside the kernel
+// its workgroup computes them one after the other as segments and stores each one's fp32 part in a slot
+// of its own (PfSk::slot); pf_fix_kernel sums a tile's parts in range order.  (Combining inside the kernel
 // -- last arriver adds -- needs the parts visible across the XCDs' L2s: per-access coherent atomics or
 // agent-scope fences on ~1 MB per tile cost more than the split saved.)  Tile index tau maps to
 // (m-tile, n-tile) so that, when there are m-tiles for all 8 XCDs, workgroup tau runs on XCD tau % 8
 // and each XCD sweeps the n-tiles of its m-tiles, keeping that activation slice in its L2.
 struct PfSk {
   int full, r, G;      // whole-tile workgroups, split tiles, ranges
-  float* part;         // workspace: two 256 KB fp32 slots per range
+  int across;          // 1 where ranges cross tiles (G no multiple of r), else 0
+  float* part;         // workspace: 256 KB fp32 slots, pf_slots(r, G) of them
+  // Slot of range g's part of split tile st.  Ranges that divide the tiles have one part each; else from
+  // one part to the next, in chunk order, the range or the tile or both go up by one, so g + st differs.
+  // (Two slots a range, one mostly unused, made smaller workspaces split less: 64 MiB, M = 768, K = 17408
+  // 257 us against 153.)
+  __device__ __forceinline__ int slot(int g, int st) const { return g + across * st; }
 };
+int64_t pf_slots(int64_t r, int64_t G) { return G % r == 0 ? G : G + r - 1; }
 
 // first chunk of range g (counted over the split tiles' chunks), and the range that holds chunk c
 __host__ __device__ __forceinline__ int pf_range_lo(int chunks, int G, int g) { return (int)((int64_t)chunks * g / G); }
@@ -463,15 +470,15 @@ __device__ __forceinline__ void pf_tile_of(int tau, int mtiles, int ntiles, int&
   }
 }
 
-// One workgroup's tile (or k-range segment of a split tile: seg >= 0, chunks [h0, h1)): the
-// prologue, the k-steps, then the epilogue or the part store.  nt: the tile's n-tile within its
+// One workgroup's tile, or (PART) k-range segment of a split tile, chunks [h0, h1): the prologue, the
+// k-steps, then the epilogue or the store of the part in slot `slot`.  nt: the tile's n-tile within its
 // matrix (or matrix pair); wkq: k-quant formats, the matrix.
-template <int EPI, int FMT>
+template <int EPI, int FMT, bool PART = false>
 __device__ __forceinline__ void pf_tile(PfLds& L, const u4_t* __restrict__ w1, const u4_t* __restrict__ w2,
                                         const uint8_t* __restrict__ wkq, const float* __restrict__ gridf,
                                         const _Float16* __restrict__ x, void* __restrict__ out,
                                         const float* __restrict__ res, int N, int K, int mt, int nt, int h0, int h1,
-                                        int seg, const PfSk& sk) {
+                                        int slot, const PfSk& sk) {
   constexpr bool kFfn = EPI == PF_FFN;
   // wave index as a scalar: the per-wave DMA selection branches on SGPRs
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -540,17 +547,17 @@ __device__ __forceinline__ void pf_tile(PfLds& L, const u4_t* __restrict__ w1, c
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // drain the clamped tail loads before the block exits
 
-  if (seg >= 0) {
+  if constexpr (PART) {
     // a segment of a split tile: store the part (the register layout, 16 B a lane, coalesced);
     // pf_fix_kernel, launched next on the stream, adds the parts in order and applies the epilogue
-    f4_t* mine = reinterpret_cast<f4_t*>(sk.part) + (size_t)seg * (kBM * kBN / 4);
+    f4_t* mine = reinterpret_cast<f4_t*>(sk.part) + (size_t)slot * (kBM * kBN / 4);
 #pragma unroll
     for (int i = 0; i < kMI; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) mine[(i * 8 + j) * kThreads + threadIdx.x] = acc[i][j];
-    return;
+  } else {
+    pf_epilogue<EPI>(acc, bg, g.m0, nt, wm, kq, col, out, res, N);
   }
-  pf_epilogue<EPI>(acc, bg, g.m0, nt, wm, kq, col, out, res, N);
 }
 
 template <int EPI>
@@ -570,11 +577,11 @@ __global__ __launch_bounds__(kThreads, 1) void pf_gemm_kernel(
   // a range's chunks [u, u1) counted over the split tiles
   const int g = bx - sk.full, u1 = pf_range_lo(sk.r * nch, sk.G, g + 1);
   int u = pf_range_lo(sk.r * nch, sk.G, g);
-  for (int slot = 2 * g; u < u1; ++slot) {
+  for (bool second = false; u < u1; second = true) {
     const int st = u / nch, h0 = u - st * nch, h1 = min(nch, h0 + (u1 - u));
     pf_tile_of(sk.full + st, mtiles, ntiles, mt, nt);
-    if (slot & 1) __syncthreads();   // the first segment's LDS is free in every wave
-    pf_tile<EPI, PF_IQ3>(L, w1, w2, nullptr, gridf, x, out, res, N, K, mt, nt, h0, h1, slot, sk);
+    if (second) __syncthreads();   // the first segment's LDS is free in every wave
+    pf_tile<EPI, PF_IQ3, true>(L, w1, w2, nullptr, gridf, x, out, res, N, K, mt, nt, h0, h1, sk.slot(g, st), sk);
     u += h1 - h0;
   }
 }
@@ -603,7 +610,7 @@ __global__ __launch_bounds__(kThreads, 1) void pfm_gemm_kernel(const PfMulti mse
   while (s + 1 < mseg.nseg && ntg >= mseg.seg[s + 1].nt0) ++s;
   const PfSeg sg = mseg.seg[s];
   const int nt = ntg - sg.nt0, nch = K / 128;
-  const PfSk none{0, 0, 0, nullptr};
+  const PfSk none{0, 0, 0, 0, nullptr};
   const u4_t* w = static_cast<const u4_t*>(sg.w);
   const uint8_t* wb = static_cast<const uint8_t*>(sg.w);
   switch (sg.fmt) {
@@ -640,15 +647,13 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out
   const int g0 = pf_range_of(chunks, sk.G, c0), g1 = pf_range_of(chunks, sk.G, c0 + nch - 1);
   constexpr size_t kSlot = kBM * kBN / 4;
   const f4_t* part = reinterpret_cast<const f4_t*>(sk.part) + (size_t)(i * 8 + jp) * kThreads + threadIdx.x;
-  // range g0 may have begun in the tile before: this tile is then its second segment
-  const int s0 = 2 * g0 + (pf_range_lo(chunks, sk.G, g0) < c0 ? 1 : 0);
   f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
   const auto add = [&](auto count, int g) {   // parts g .. g + count - 1, all requested first
     constexpr int C = decltype(count)::value;
     f4_t v[C][2];
 #pragma unroll
     for (int q = 0; q < C; ++q) {
-      const f4_t* p = part + (size_t)(g + q == g0 ? s0 : 2 * (g + q)) * kSlot;
+      const f4_t* p = part + (size_t)sk.slot(g + q, st) * kSlot;
       v[q][0] = p[0];
       v[q][1] = p[4 * kThreads];
     }
@@ -691,18 +696,18 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out
 // one more round of whole tiles.  Cost in 1/40 chunk (0.1 us; a 128-k chunk of a tile takes about 4 us a
 // CU): the longest range's chunks, 1.5 chunks a segment for its prologue, 1 a part (256 KB written and
 // read again).  Measured, the FFN block (G by equal splits of 2 to 4 a tile -> by this rule): M = 256
-// 284 -> 198 us (down: 80 workgroups -> 240).  With G always one a CU M = 1536 took 873 us against 862.
+// 284 -> 188 us (down: 80 workgroups -> 240).  With G always one a CU M = 1536 took 873 us against 862.
 int pf_ranges(int r, int nch, int G0, int64_t slots) {
   const int64_t chunks = (int64_t)r * nch;
   int best = 0;
   int64_t least = 40LL * nch;
-  const auto take = [&](int64_t G, int64_t segs, int64_t parts, int64_t need) {
-    if (G <= r || 4 * G > chunks || need > slots) return;
+  const auto take = [&](int64_t G, int64_t segs, int64_t parts) {
+    if (G <= r || 4 * G > chunks || pf_slots(r, G) > slots) return;
     const int64_t cost = 40 * ((chunks + G - 1) / G) + 60 * segs + parts;
     if (cost < least) { least = cost; best = (int)G; }
   };
-  for (int64_t G = 2 * (int64_t)r; G <= G0; G += r) take(G, 1, G, 2 * G);
-  take(G0, 2, r + G0 - 1, 2 * (int64_t)G0);
+  for (int64_t G = 2 * (int64_t)r; G <= G0; G += r) take(G, 1, G);
+  take(G0, 2, r + G0 - 1);
   return best;
 }
 
@@ -711,7 +716,7 @@ int pf_launch(const u4_t* w1, const u4_t* w2, const float* gridf, const _Float16
               int M, int N, int K, int mtiles, int ntiles, hipStream_t st) {
   const int tiles = mtiles * ntiles, G0 = tlx_cu_count(), nch = K / 128;
   const int R = tiles / G0, r = tiles - R * G0;
-  PfSk sk{tiles, 0, 0, nullptr};
+  PfSk sk{tiles, 0, 0, 0, nullptr};
   if (r > 0) {
     void* ws = nullptr;
     size_t wsb = 0;
@@ -719,7 +724,7 @@ int pf_launch(const u4_t* w1, const u4_t* w2, const float* gridf, const _Float16
     TLX_RET_IF(rc != TLX_OK, rc);
     const int64_t slots = ws != nullptr ? (int64_t)(std::min(wsb, kPfPartBytes) / (kBM * kBN * 4)) : 0;
     const int G = pf_ranges(r, nch, G0, slots);
-    if (G > 0) sk = PfSk{R * G0, r, G, static_cast<float*>(ws)};
+    if (G > 0) sk = PfSk{R * G0, r, G, G % r != 0, static_cast<float*>(ws)};
   }
   pf_gemm_kernel<EPI><<<sk.full + sk.G, kThreads, 0, st>>>(w1, w2, gridf, x, out, res, M, N, K, mtiles, ntiles, sk);
   if (sk.G > 0) {
