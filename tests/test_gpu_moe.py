@@ -141,9 +141,9 @@ def test_moe_route(gpu):
     np.testing.assert_allclose(sg.cpu().numpy(), ref_sg, rtol=1e-5)
 
 
-@pytest.mark.parametrize("P", [1, 3, 4, 5, 96, 97, 257, 1027])
+@pytest.mark.parametrize("P", [1, 3, 4, 5, 80, 81, 96, 97, 257, 1027])
 def test_moe_route_batches(gpu, P):
-    """A workgroup per router row (up to 96 positions; fewer than, as many as and more than its four
+    """A workgroup per router row (up to 80 positions; fewer than, as many as and more than its four
     waves), and every positions-a-workgroup form (1, 4, 8) with a ragged last workgroup: logits in float64 decide
     the ids where the 8th and 9th are apart by more than fp32 sums of 2048 terms can move (1e-4)."""
     print(f"[case] moe route P={P}", flush=True)
@@ -188,6 +188,84 @@ def test_moe_topk_extremes(gpu):
     np.testing.assert_allclose(gates.cpu().numpy(), ref_g, rtol=2e-6, atol=1e-7)
     ops.moe_topk(torch.full((1, moe.E), float("nan"), device=gpu), eids[:1], gates[:1])
     assert eids[0].tolist() == list(range(8)) and gates[0].isnan().all()   # eight different experts
+
+
+@pytest.mark.parametrize("P", [1, 5, 80, 96])
+def test_moe_route_forms_agree(gpu, P):
+    """The router's results are the same bits on every route: the current stream (given or not), another
+    stream, a caller's logits buffer, stream capture (the replays, eager work between them) and the C call.
+    Nothing is allocated under capture, on another stream, or with a logits buffer."""
+    print(f"[case] moe route forms P={P}", flush=True)
+    rng = np.random.default_rng(1400 + P)
+    wrt = torch.from_numpy((rng.standard_normal((moe.E, moe.HID)) * 0.02).astype(np.float32)).to(gpu)
+    wsh = torch.from_numpy((rng.standard_normal(moe.HID) * 0.02).astype(np.float32)).to(gpu)
+    h = torch.from_numpy(rng.standard_normal((P, moe.HID)).astype(np.float32)).to(gpu)
+    outs = lambda: (torch.zeros(P, 8, dtype=torch.int16, device=gpu), torch.zeros(P, 8, device=gpu), torch.zeros(P, device=gpu))
+    allocs = lambda: torch.cuda.memory_stats(gpu)["allocation.all.allocated"]
+    cur, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    logits = torch.empty(P, moe.E, device=gpu)
+    ref = outs()
+    ops.moe_route(wrt, wsh, h, *ref)
+    got = {}
+
+    def run(name, alloc, **kw):
+        o = got[name] = outs()
+        torch.cuda.synchronize()
+        before = allocs()
+        ops.moe_route(wrt, wsh, h, *o, **kw)
+        assert alloc or allocs() == before, name
+        torch.cuda.synchronize()
+
+    run("current stream given", True, stream=cur)
+    run("its handle given", True, stream=cur.cuda_stream)
+    run("another stream", False, stream=side)
+    run("another stream, logits", False, stream=side, logits=logits)
+    run("logits", False, logits=logits)
+    o = got["C call"] = outs()
+    call("tlx_moe_route", wrt.data_ptr(), wsh.data_ptr(), h.data_ptr(), *(t.data_ptr() for t in o), P, cur.cuda_stream)
+    for name, kw in (("capture", {}), ("capture, logits", {"logits": logits})):
+        o = got[name] = outs()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            before = allocs()
+            ops.moe_route(wrt, wsh, h, *o, **kw)
+            assert allocs() == before, name
+        for _ in range(3):
+            for t in o:
+                t.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(o, ref)), name
+            ops.moe_route(wrt, wsh, h, *outs())
+    torch.cuda.synchronize()
+    for name, o in got.items():
+        assert all(torch.equal(a, b) for a, b in zip(o, ref)), name
+    # the largest batches' form: the same positions among more give the same bits
+    big = torch.randn(1100, moe.HID, device=gpu)
+    big[1000:1000 + P] = h
+    o = (torch.zeros(1100, 8, dtype=torch.int16, device=gpu), torch.zeros(1100, 8, device=gpu), torch.zeros(1100, device=gpu))
+    for n in (300, 1100):   # 4 and 8 positions a workgroup
+        ops.moe_route(wrt, wsh, big[1100 - n:].contiguous(), *o)
+        at = n - 100
+        assert all(torch.equal(a[at:at + P], b) for a, b in zip(o, ref)), n
+
+
+def test_moe_route_logits_arguments(gpu):
+    print("[case] moe route logits arguments", flush=True)
+    wrt, wsh, h = torch.zeros(moe.E, moe.HID, device=gpu), torch.zeros(moe.HID, device=gpu), torch.zeros(2, moe.HID, device=gpu)
+    o = (torch.zeros(2, 8, dtype=torch.int16, device=gpu), torch.zeros(2, 8, device=gpu), torch.zeros(2, device=gpu))
+    lg = torch.zeros(3, moe.E, device=gpu)
+    with pytest.raises(ValueError):   # logits of one position for two
+        ops.moe_route(wrt, wsh, h, *o, logits=lg[:1])
+    with pytest.raises(ValueError):   # logits on the host
+        ops.moe_route(wrt, wsh, h, *o, logits=lg.cpu())
+    ptr = [t.data_ptr() for t in (wrt, wsh, h, lg) + o]
+    for bad in ({0: 4}, {1: 4}, {2: 8}, {3: 4}):   # misaligned wrt, wsh, h, logits
+        with pytest.raises(TlxError):
+            call("tlx_moe_route_logits", *(p + bad.get(i, 0) for i, p in enumerate(ptr)), 2, None)
+    with pytest.raises(TlxError):
+        call("tlx_moe_route_logits", *ptr, 0, None)
 
 
 def test_moe_route_given_stream(gpu):

@@ -48,17 +48,47 @@ __device__ __forceinline__ float wave_max(float v) {   // (fmaxf: NaN only if ev
   v = fmaxf(v, dpp_f<0x143, 0xC>(v));   // row_bcast:31 into rows 2 and 3
   return lane63(v);
 }
-__device__ __forceinline__ float wave_sum(float v) {
+// The order of a router row's sum (fp32 products and sums), the same in both kernels below, so that a
+// logit's bits depend on neither: 64 chains of 8 steps a component -- chain (j, piece), j < 16, piece < 4,
+// takes the row's 16-B pieces 32 j + 4 i + piece, i = 0 .. 7 -- then chains j in fours, the four sums of
+// those, and last the pieces.
+constexpr int kRtChain = 8;
+__device__ __forceinline__ void rt_step(float4& acc, float4 w, float4 x, bool first) {
+  acc.x = first ? w.x * x.x : __builtin_fmaf(w.x, x.x, acc.x);
+  acc.y = first ? w.y * x.y : __builtin_fmaf(w.y, x.y, acc.y);
+  acc.z = first ? w.z * x.z : __builtin_fmaf(w.z, x.z, acc.z);
+  acc.w = first ? w.w * x.w : __builtin_fmaf(w.w, x.w, acc.w);
+}
+__device__ __forceinline__ float rt_fold(float4 acc) { return (acc.x + acc.y) + (acc.z + acc.w); }
+__device__ __forceinline__ float rt_pieces(float v) {   // over the four lanes of a quad
   v += dpp_f<0xB1, 0xF>(v);
   v += dpp_f<0x4E, 0xF>(v);
-  v += dpp_f<0x141, 0xF>(v);
-  v += dpp_f<0x140, 0xF>(v);
-  const float r15 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));
-  v += r15;   // (0 in rows 0 and 2)
-  const float r31 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));
-  v += r31;
-  return lane63(v);
+  return v;
 }
+// a row's sum by a wave, lane 4 j + piece holding that chain's pieces of the row and of the position;
+// valid in lanes 0 .. 3
+__device__ __forceinline__ float rt_row(const float4 (&w)[kRtChain], const float4 (&x)[kRtChain]) {
+  float4 acc;
+#pragma unroll
+  for (int i = 0; i < kRtChain; ++i) rt_step(acc, w[i], x[i], i == 0);
+  const float q = rt_fold(acc);
+  float g = q + dpp_f<0x104, 0xF>(q);   // row_shl: lane l takes lane l + 4, + 8, + 12 of its 16-lane row
+  g += dpp_f<0x108, 0xF>(q);
+  g += dpp_f<0x10C, 0xF>(q);
+  const uint32_t gb = __builtin_bit_cast(uint32_t, g);
+  const auto r = __builtin_amdgcn_permlane16_swap(gb, gb, false, false);   // row 0: rows 0 and 1; row 2: rows 2 and 3
+  const uint32_t r0 = r[0], r1 = r[1];   // (values of their own: __builtin_bit_cast of a vector's element takes element 0)
+  const uint32_t r2 = __builtin_amdgcn_permlane32_swap(r0, r0, false, false)[1];   // row 0: row 2's
+  const uint32_t r3 = __builtin_amdgcn_permlane32_swap(r1, r1, false, false)[1];
+  const float v = ((__builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1)) + __builtin_bit_cast(float, r2)) + __builtin_bit_cast(float, r3);
+  return rt_pieces(v);
+}
+// 16-B piece k4 of wsh, which is 8-B aligned
+__device__ __forceinline__ float4 rt_wsh(const float* wsh, int k4) {
+  const float2 a = reinterpret_cast<const float2*>(wsh)[2 * k4], b = reinterpret_cast<const float2*>(wsh)[2 * k4 + 1];
+  return float4{a.x, a.y, b.x, b.y};
+}
+__device__ __forceinline__ float rt_gate(float v) { return 1.f / (1.f + expf(-v)); }
 
 // Top-8 of one position by a wave, lane l holding experts 4 l .. 4 l + 3 in v: 8 passes, each the
 // wave's largest value and, among the experts that equal it, the lowest id (the first lane of a
@@ -108,21 +138,20 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
 // rt8e256: logits = wrt . h, shared gate sg = sigmoid(wsh . h), then the top-8.  A 16-wave workgroup
 // takes NP positions: their h in LDS, wave w the 16 experts 16 w .. , four lanes a row so that a
 // wave's 16-B loads read 64 contiguous bytes a quad (a row per lane, as before, took a quarter of
-// that rate), 16 or 8 loads ahead; every weight feeds NP positions.  Products and sums are fp32: 16 fixed
-// partial sums of 128 terms a logit.  The bound at few positions is the 2 MB of wrt through one
-// CU's load path (64 B a clock), at many the fp32 FMAs.
-constexpr int kRtThreads = 1024;
+// that rate), 16 or 8 loads ahead; every weight feeds NP positions.  The bound at few positions is the
+// 2 MB of wrt through one CU's load path (64 B a clock), at many the reads of h from LDS (16 B a wave and
+// step for 4 FMAs).
+constexpr int kRtThreads = 1024, kRtWaves = kRtThreads / TLX_WAVE;
 template <int NP>
 __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
                                                                const float* __restrict__ h, uint16_t* __restrict__ eids,
                                                                float* __restrict__ gates, float* __restrict__ sg, int P) {
   __shared__ float4 hs[NP][kHid / 4];
   __shared__ float4 lg[NP][kE / 4];
-  __shared__ float shp[NP][kRtThreads / TLX_WAVE];
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, p0 = blockIdx.x * NP;
   const int row = 16 * wave + (lane >> 2), piece = lane & 3;
   constexpr int kSteps = kHid / 16;   // 16 k a step
-  constexpr int kRtAhead = NP <= 4 ? 16 : 8;   // as the sums leave room (P = 2048: 48.8 us at 16, 43.6 at 8)
+  constexpr int kRtAhead = NP <= 4 ? 16 : 8;   // as the sums leave room (8 for NP = 4: P = 300 22.4 -> 23.8 us)
   const float4* wr = reinterpret_cast<const float4*>(wrt + (size_t)row * kHid) + piece;
   float4 w[kRtAhead];
 #pragma unroll
@@ -131,51 +160,57 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __re
     const int p = i / (kHid / 4), k4 = i % (kHid / 4);
     hs[p][k4] = reinterpret_cast<const float4*>(h + (size_t)min(p0 + p, P - 1) * kHid)[k4];   // past P: unused
   }
-  const float2 ws = reinterpret_cast<const float2*>(wsh)[t];
   __syncthreads();
-  float4 acc[NP];
+  float four[NP], tot[NP];   // the sums of the chains of the present four, and of the fours before
 #pragma unroll
-  for (int p = 0; p < NP; ++p) acc[p] = float4{0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < NP; ++p) four[p] = tot[p] = 0.f;
   // slot u of the ring: step s0 + u's weights, then (once used) step s0 + kRtAhead + u's.  The fences
   // keep each pair of steps' requests behind its uses: without them the scheduler moves the requests
   // to where the loop's end has to wait for all of them.
   for (int s0 = 0; s0 < kSteps; s0 += kRtAhead) {
     const float4* wn = wr + 4 * min(s0 + kRtAhead, kSteps - kRtAhead);   // past the end: the last steps again
+    float4 acc[NP];
 #pragma unroll
     for (int u = 0; u < kRtAhead; ++u) {
       const float4 wv = w[u];
 #pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        const float4 x = hs[p][4 * (s0 + u) + piece];
-        acc[p].x += wv.x * x.x;
-        acc[p].y += wv.y * x.y;
-        acc[p].z += wv.z * x.z;
-        acc[p].w += wv.w * x.w;
-      }
+      for (int p = 0; p < NP; ++p) rt_step(acc[p], wv, hs[p][4 * (s0 + u) + piece], u % kRtChain == 0);
       w[u] = wn[4 * u];
       if (u & 1) __builtin_amdgcn_sched_barrier(0);
+      if (u % kRtChain == kRtChain - 1) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) four[p] += rt_fold(acc[p]);
+      }
+    }
+    if ((s0 + kRtAhead) % (4 * kRtChain) == 0) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        tot[p] += four[p];
+        four[p] = 0.f;
+      }
     }
   }
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    float v = (acc[p].x + acc[p].y) + (acc[p].z + acc[p].w);
-    v += dpp_f<0xB1, 0xF>(v);
-    v += dpp_f<0x4E, 0xF>(v);
+    const float v = rt_pieces(tot[p]);
     if (piece == 0) reinterpret_cast<float*>(lg[p])[row] = v;
-    const float2 x = reinterpret_cast<const float2*>(hs[p])[t];
-    const float s = wave_sum(ws.x * x.x + ws.y * x.y);
-    if (lane == 0) shp[p][wave] = s;
   }
   __syncthreads();
+  // the first NP waves a position's top-8, the last NP a position's shared gate
+  static_assert(2 * NP <= kRtWaves, "");
+  const int ps = kRtWaves - 1 - wave;
   if (wave < NP && p0 + wave < P) {
-    const int p = p0 + wave;
-    topk8_wave(lg[wave][lane], lane, eids + (size_t)p * kTopK, gates + (size_t)p * kTopK);
-    if (lane == 0) {
-      float s = 0.f;
+    topk8_wave(lg[wave][lane], lane, eids + (size_t)(p0 + wave) * kTopK, gates + (size_t)(p0 + wave) * kTopK);
+  } else if (ps < NP && p0 + ps < P) {
+    float4 a[kRtChain], x[kRtChain];
 #pragma unroll
-      for (int i = 0; i < kRtThreads / TLX_WAVE; ++i) s += shp[wave][i];
-      sg[p] = 1.f / (1.f + expf(-s));
+    for (int i = 0; i < kRtChain; ++i) {
+      const int k4 = 32 * (lane >> 2) + 4 * i + piece;
+      a[i] = rt_wsh(wsh, k4);
+      x[i] = hs[ps][k4];
     }
+    const float v = rt_row(a, x);
+    if (lane == 0) sg[p0 + ps] = rt_gate(v);
   }
 }
 
@@ -183,47 +218,37 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __re
 // positions dealt to its four waves: a wave holds the row's 8 KB in 32 registers and reads each
 // position's h against it, two positions in flight.  wrt then comes through every CU's load path
 // instead of one CU's per position; the logits go through memory to moe_topk_kernel.  Both launches, us
-// at P = 1 / 4 / 16 / 64 / 128: 5.7 / 6.5 / 8.8 / 15.9 / 24.9 (1 wave 5.6 / 6.9 / 12.2 / 31 / 57, 8 waves
-// 5.5 / 6.4 / 9.2 / 15.3 / 23.5) against 21.2 / 23.1 / 23.5 / 22.7 / 22.7 of moe_route_kernel.  Bound by the two
-// launches at few positions, from 16 on by h, which every workgroup reads whole (8 KB a position and CU).
+// at P = 1 / 4 / 16 / 64 / 80 / 96: 5.1 / 6.0 / 8.1 / 15.1 / 17.4 / 19.8 against 17.1 / 17.3 / 17.5 / 17.5 / 17.6 /
+// 17.6 of moe_route_kernel (one session, replayed back to back).  Other wave counts, measured at P = 1 / 4 / 16 /
+// 64 / 128 with another order of the sums: 1 wave 5.6 / 6.9 / 12.2 / 31 / 57, 4 waves 5.7 / 6.5 / 8.8 / 15.9 / 24.9,
+// 8 waves 5.5 / 6.4 / 9.2 / 15.3 / 23.5.  Bound by the two launches at few positions, from 16 on by h, which
+// every workgroup reads whole (8 KB a position and CU).  The sum of a position's chains beside the products of
+// the next position's: 14.7 at P = 64, but 6.2 / 8.2 at 4 / 16.
 constexpr int kLgWaves = 4;
 __global__ __launch_bounds__(kLgWaves * TLX_WAVE) void moe_logits_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
                                                                          const float* __restrict__ h, float* __restrict__ logits,
                                                                          float* __restrict__ sg, int P) {
   const int row = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  constexpr int kPer = kHid / 4 / TLX_WAVE;
-  const float4* hp = reinterpret_cast<const float4*>(h) + lane;
-  float4 w[kPer], x[kPer];
+  const int k0 = 32 * (lane >> 2) + (lane & 3);   // (a quad's loads are 64 contiguous bytes)
+  const float4* hp = reinterpret_cast<const float4*>(h) + k0;
+  float4 w[kRtChain], x[kRtChain];
   if (wave >= P) return;
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int k4 = TLX_WAVE * i + lane;
-    if (row < kE) {
-      w[i] = reinterpret_cast<const float4*>(wrt + (size_t)row * kHid)[k4];
-    } else {   // (wsh is 8-B aligned)
-      const float2 a = reinterpret_cast<const float2*>(wsh)[2 * k4], b = reinterpret_cast<const float2*>(wsh)[2 * k4 + 1];
-      w[i] = float4{a.x, a.y, b.x, b.y};
-    }
-  }
+  for (int i = 0; i < kRtChain; ++i)
+    w[i] = row < kE ? reinterpret_cast<const float4*>(wrt + (size_t)row * kHid)[k0 + 4 * i] : rt_wsh(wsh, k0 + 4 * i);
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) x[i] = hp[(size_t)wave * (kHid / 4) + TLX_WAVE * i];
+  for (int i = 0; i < kRtChain; ++i) x[i] = hp[(size_t)wave * (kHid / 4) + 4 * i];
   for (int p = wave; p < P; p += kLgWaves) {
     const float4* hn = hp + (size_t)min(p + kLgWaves, P - 1) * (kHid / 4);   // past the end: the last position again
-    float4 n[kPer], s = float4{0.f, 0.f, 0.f, 0.f};
+    float4 n[kRtChain];
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) n[i] = hn[TLX_WAVE * i];
+    for (int i = 0; i < kRtChain; ++i) n[i] = hn[4 * i];
+    const float v = rt_row(w, x);
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      s.x += w[i].x * x[i].x;
-      s.y += w[i].y * x[i].y;
-      s.z += w[i].z * x[i].z;
-      s.w += w[i].w * x[i].w;
-      x[i] = n[i];
-    }
-    const float v = wave_sum((s.x + s.y) + (s.z + s.w));
+    for (int i = 0; i < kRtChain; ++i) x[i] = n[i];
     if (lane == 0) {
       if (row < kE) logits[(size_t)p * kE + row] = v;
-      else sg[p] = 1.f / (1.f + expf(-v));
+      else sg[p] = rt_gate(v);
     }
   }
 }
@@ -1220,9 +1245,9 @@ extern "C" int tlx_moe_topk(const float* logits, uint16_t* eids, float* gates, i
 }
 
 // Positions a workgroup by batch, the fewest that keep the grid within one workgroup a CU (256):
-// us at 1 / 4 / 8 positions a workgroup: P = 4 22.9 / 29.2 / 44.6, 256 24.0 / 27.7 / 45.3, 300 39.9 /
-// 27.5 / 45.3, 1024 77.9 / 29.8 / 45.6, 1500 112 / 50.2 / 45.5, 2048 148 / 57.3 / 43.6.  (A row per lane
-// and one position a workgroup: 75 us at P = 4.)
+// us at 1 / 4 / 8 positions a workgroup: P = 4 17.4 / 21.7 / 42.2, 256 20.7 / 22.3 / 43.3, 300 35.4 /
+// 22.5 / 43.5, 1024 74 / 29.8 / 44.5, 1100 89 / 47.3 / 44.7, 2048 147 / 56.3 / 47.3.  (A row per lane and one
+// position a workgroup: 62 us at P = 4, 525 at 2048.)
 constexpr int kRt1 = 256, kRt4 = 1024;
 
 extern "C" int tlx_moe_route(const float* wrt, const float* wsh, const float* h, uint16_t* eids, float* gates,

@@ -3,8 +3,8 @@
 Each function keeps the reference kernel's name and positional argument order
 (``ffn8(wg, wu, gridf, hhx, gact)`` etc., /root/reference/engine/ffn8.cu:134-136) and takes
 torch tensors on the GPU.  Sizes the reference bakes into kernel names (M, N, K) are read
-from the tensor shapes.  Like the reference, the output buffers are caller-owned; nothing is
-allocated here.  Errors raise ``TlxError`` (the reference asserts in Python).
+from the tensor shapes.  Like the reference, the output buffers are caller-owned; the calls allocate
+nothing (but the router's logits, where none are given: moe_route).  Errors raise ``TlxError`` (the reference asserts in Python).
 """
 import torch
 
@@ -61,8 +61,8 @@ def _ws(t):
 
 
 def _stream(stream):
-    if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+    if stream is None:   # (the device given: 2.9 -> 1.5 us of a call's host time)
+        return torch.cuda.current_stream(torch.cuda.current_device()).cuda_stream
     return getattr(stream, "cuda_stream", stream)
 
 
@@ -631,13 +631,18 @@ def moe_topk(logits, eids, gates, stream=None):
     call("tlx_moe_topk", logits.data_ptr(), eids.data_ptr(), gates.data_ptr(), logits.shape[0], _stream(stream))
 
 
-# Largest batch the router takes with a workgroup per router row and the logits in memory: at 64
-# positions 15.9 us against 22.7 with whole positions a workgroup, at 128 24.9 against 22.7.
-MOE_ROUTE_LOGITS_MAX_P = 96
+# Largest batch the router takes with a workgroup per router row and the logits in memory: device time
+# at 64 / 80 / 96 positions 15.1 / 17.4 / 19.8 us against 17.5 / 17.6 / 17.6 with whole positions a workgroup.
+MOE_ROUTE_LOGITS_MAX_P = 80
 
 
-def moe_route(wrt, wsh, h, eids, gates, sg, stream=None):
-    """rt8e256(wrt, wsh, h, eids, gates, sg)."""
+def moe_route(wrt, wsh, h, eids, gates, sg, stream=None, logits=None):
+    """rt8e256(wrt, wsh, h, eids, gates, sg).
+
+    Up to MOE_ROUTE_LOGITS_MAX_P positions the faster form passes the logits through memory: f32[P][256],
+    the caller's ``logits`` if given (written), else a tensor of torch's allocator where its lifetime is the
+    call's -- on the current stream, outside stream capture.  Elsewhere, and above, nothing is allocated and
+    the form without them runs.  Both sum in the same order: the results are the same bits."""
     P = h.shape[0]
     _need(wrt, 256 * 2048 * 4, "wrt")
     _need(wsh, 2048 * 4, "wsh")
@@ -646,14 +651,19 @@ def moe_route(wrt, wsh, h, eids, gates, sg, stream=None):
     _need(gates, P * 8 * 4, "gates")
     _need(sg, P * 4, "sg")
     _dev(wrt, wsh, h, eids, gates, sg)
-    # (the logits belong to the current stream; a call on another one takes the form without them)
-    if stream is None and 0 < P <= MOE_ROUTE_LOGITS_MAX_P:
-        logits = torch.empty(P, 256, dtype=torch.float32, device=h.device)
-        call("tlx_moe_route_logits", wrt.data_ptr(), wsh.data_ptr(), h.data_ptr(), logits.data_ptr(), eids.data_ptr(),
-             gates.data_ptr(), sg.data_ptr(), P, _stream(None))
-        return
+    if logits is not None:
+        _need(logits, P * 256 * 4, "logits")
+        _dev(logits)
+    st = _stream(stream)
+    if 0 < P <= MOE_ROUTE_LOGITS_MAX_P:
+        if logits is None and (stream is None or st == _stream(None)) and not torch.cuda.is_current_stream_capturing():
+            logits = torch.empty(P, 256, dtype=torch.float32, device="cuda")   # the current device: that stream's
+        if logits is not None:
+            call("tlx_moe_route_logits", wrt.data_ptr(), wsh.data_ptr(), h.data_ptr(), logits.data_ptr(),
+                 eids.data_ptr(), gates.data_ptr(), sg.data_ptr(), P, st)
+            return
     call("tlx_moe_route", wrt.data_ptr(), wsh.data_ptr(), h.data_ptr(), eids.data_ptr(), gates.data_ptr(),
-         sg.data_ptr(), h.shape[0], _stream(stream))
+         sg.data_ptr(), P, st)
 
 
 def moe_max_items(npair):
