@@ -171,23 +171,38 @@ def test_moe_route_batches(gpu, P):
 
 
 def test_moe_topk_extremes(gpu):
-    """Ties over every lane, infinities and the mask's own value: the oracle's ids (lower id first)."""
+    """Ties over every lane, infinities, the mask's own value and rows with fewer than 8 values above
+    it: the oracle's ids (lower id first; a chosen id again where nothing else is left)."""
     print("[case] moe topk extremes", flush=True)
-    lg = np.zeros((5, moe.E), np.float32)                     # all equal: ids 0..7
+    low = np.float32(-3.402823466e38)                         # the mask
+    lg = np.zeros((12, moe.E), np.float32)                    # all equal: ids 0..7
     lg[1] = -np.arange(moe.E)                                 # one lane holds the first four
     lg[2] = np.arange(moe.E)[::-1] // 3                       # ties of three across lanes
     lg[3, ::2], lg[3, 1::2] = -0.0, 0.0                       # zeros of both signs are equal
     lg[4] = -3.0e38
     lg[4, 255] = 3.0e38
-    eids = torch.empty(5, 8, dtype=torch.int16, device=gpu)
-    gates = torch.empty(5, 8, device=gpu)
+    lg[5], lg[5, [9, 200]] = np.arange(moe.E), np.inf         # two infinities: NaN gates
+    lg[6] = -np.inf                                           # nothing but -inf
+    lg[7], lg[7, [3, 77, 78, 250]] = -np.inf, [1.0, 3.0, 3.0, 2.0]   # four numbers among -inf
+    lg[8] = low                                               # the mask's value everywhere
+    lg[9], lg[9, [60, 61, 190]] = low, [0.5, -1.0, 0.5]       # three numbers above it
+    lg[10], lg[10, 255] = -np.inf, low                        # the mask's value among -inf
+    lg[11, :250], lg[11, 250:] = -np.inf, -np.arange(6)       # six numbers at the end
+    eids = torch.empty(12, 8, dtype=torch.int16, device=gpu)
+    gates = torch.empty(12, 8, device=gpu)
     ops.moe_topk(torch.from_numpy(lg).to(gpu), eids, gates)
     torch.cuda.synchronize()
-    ref_e, ref_g = moe.topk_ref(lg)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref_e, ref_g = moe.topk_ref(lg)
     assert np.array_equal(eids.cpu().numpy().view(np.uint16), ref_e)
     np.testing.assert_allclose(gates.cpu().numpy(), ref_g, rtol=2e-6, atol=1e-7)
     ops.moe_topk(torch.full((1, moe.E), float("nan"), device=gpu), eids[:1], gates[:1])
     assert eids[0].tolist() == list(range(8)) and gates[0].isnan().all()   # eight different experts
+    few = torch.full((1, moe.E), float("nan"), device=gpu)
+    few[0, [10, 20, 30]] = torch.tensor([1.0, 2.0, 3.0], device=gpu)
+    ops.moe_topk(few, eids[:1], gates[:1])   # the numbers, then the lowest of their ids with gate 0
+    assert eids[0].tolist() == [30, 20] + [10] * 6 and (gates[0, 3:] == 0).all()
+    torch.testing.assert_close(gates[0, :3].cpu(), torch.softmax(torch.tensor([3.0, 2.0, 1.0]), 0), rtol=2e-6, atol=0)
 
 
 @pytest.mark.parametrize("P", [1, 5, 80, 96])

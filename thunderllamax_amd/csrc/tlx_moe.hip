@@ -94,8 +94,10 @@ __device__ __forceinline__ float rt_gate(float v) { return 1.f / (1.f + expf(-v)
 // wave's largest value and, among the experts that equal it, the lowest id (the first lane of a
 // ballot, then its first element: scalar work), which is masked for the passes after.  A pass is 9
 // dependent vector steps and four compares; exchanging (value, id) pairs lane by lane took 15 + 4
-// compare-and-select pairs a pass on a 16-lane row.  Softmax over the 8, summed in pass order.  A
-// NaN is never chosen before a number (a position of NaNs takes ids 0, 1, .. and NaN gates).
+// compare-and-select pairs a pass on a 16-lane row.  Softmax over the 8, summed in pass order.  The
+// mask is the lowest finite value, as the reference's: where fewer than 8 logits lie above it (the rest
+// -inf, the mask's own value or NaN) the passes left take the lowest id already chosen again, with a gate
+// of 0 beside larger ones.  A position of NaNs alone takes ids 0 .. 7 and NaN gates.
 __device__ __forceinline__ void topk8_wave(float4 in, int lane, uint16_t* eids, float* gates) {
   float v[4] = {in.x, in.y, in.z, in.w};
   int id = 0;
