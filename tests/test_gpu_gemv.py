@@ -357,7 +357,11 @@ def test_attention_variants(gpu, name, M):
 @pytest.mark.parametrize("K,Nq,Nk,Nv,M,v4,raw", [
     (512, 4009, 250, 1003, 3, True, False), (512, 16, 4500, 9, 16, False, False),
     (2560, 100, 17, 5000, 7, True, True), (5120, 33, 40, 24, 12, True, False),
-    (5120, 33, 40, 24, 13, False, False), (256, 16, 16, 16, 1, True, True)])
+    (5120, 33, 40, 24, 13, False, False), (256, 16, 16, 16, 1, True, True),
+    # a launch a matrix, where q's rows fit the LDS with more activation rows than the three together do
+    # (K = 4096: 16 against 15; 8192: 8 against 7)
+    (4096, 70, 40, 33, 16, True, True), (4096, 70, 40, 33, 16, False, False),
+    (8192, 40, 24, 50, 8, False, False), (8192, 40, 24, 50, 9, True, False)])
 def test_qkv_three_formats_one_launch(gpu, K, Nq, Nk, Nv, M, v4, raw):
     from thunderllamax_amd._lib import V_Q4K
     print(f"[case] q6/iq3/q4 K={K} rows {Nq} {Nk} {Nv} M={M} v4={v4} raw={raw}", flush=True)
