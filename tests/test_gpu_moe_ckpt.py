@@ -429,12 +429,13 @@ def test_ckpt_argument_validation(gpu, ckpt):
              16385, LAYOUT_TILED, None)
 
 
-@pytest.mark.parametrize("P", [11, 300])
-def test_ckpt_layer(gpu, ckpt, P):
-    """ops.moe_layer_ckpt (top-8, pair walk at P=11 / sort + grouped forms at P=300, IQ3_S up,
+@pytest.mark.parametrize("P,lay", [(11, LAYOUT_RAW), (300, LAYOUT_RAW), (17, LAYOUT_TILED), (32, LAYOUT_RAW),
+                                   (33, LAYOUT_RAW), (40, LAYOUT_TILED), (41, LAYOUT_TILED)])
+def test_ckpt_layer(gpu, ckpt, ckpt_tiled, P, lay):
+    """ops.moe_layer_ckpt (top-8, pair walk up to P=32, 40 on tiled slabs / sort + grouped forms above, IQ3_S up,
     Q6_K down, Q8_0 shared, combine): every pair's act / parts and the shared expert against the
     oracle, y against the combine of the GPU's own parts and shared output."""
-    print(f"[case] checkpoint-class MoE layer P={P}", flush=True)
+    print(f"[case] checkpoint-class MoE layer P={P} layout={lay}", flush=True)
     rng = np.random.default_rng(47 + P)
     x = synth.bf16_round(0.05 * rng.standard_normal((P, moe.HID)).astype(np.float32))
     logits = rng.standard_normal((P, moe.E)).astype(np.float32)
@@ -442,9 +443,13 @@ def test_ckpt_layer(gpu, ckpt, P):
     hres = rng.standard_normal((P, moe.HID)).astype(np.float32)
     sc = ops.MoeScratch(P, gpu)
     y = torch.empty(P, moe.HID, dtype=torch.float32, device=gpu)
+    slabs = ckpt if lay == LAYOUT_RAW else ckpt_tiled
+    sc.eoff.fill_(-1)   # the sort's output: the pair walk leaves it
     ops.moe_layer_ckpt(torch.from_numpy(logits).to(gpu), torch.from_numpy(sg).to(gpu), torch.from_numpy(x).to(gpu),
-                       torch.from_numpy(hres).to(gpu), y, ckpt["ptbl"], ckpt["ptbl_dn"], ckpt["dsh"], ckpt["gridf"], sc)
+                       torch.from_numpy(hres).to(gpu), y, slabs["ptbl"], slabs["ptbl_dn"], ckpt["dsh"], ckpt["gridf"], sc,
+                       layout=lay)
     torch.cuda.synchronize()
+    assert (sc.eoff[256].item() == -1) == (P <= (32 if lay == LAYOUT_RAW else 40))
     eids, gates = moe.topk_ref(logits)
     assert np.array_equal(sc.eids.cpu().numpy().view(np.uint16), eids)
     act, parts, shared = sc.act.cpu().numpy(), sc.parts.cpu().numpy(), sc.shared.cpu().numpy()

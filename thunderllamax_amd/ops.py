@@ -1018,8 +1018,12 @@ _SIDE_STREAMS = {}
 # launch it skips costs more than the expert slabs that two pairs of the batch share and the
 # pair walk reads twice.
 MOE_PAIR_WALK_MAX_P = 16
-# The same for the checkpoint's classes with a Q6_K down: layer, pair walk against sorted forms, tiled
-# slabs P = 32 109 / 151 us, 40 131 / 156, 48 154 / 159; GGUF rows 32 151 / 167, 40 184 / 171.
+# The same for the checkpoint's classes with a Q6_K down, by the layout: where the lines lie for uniform
+# routing.  Layer, us, pair walk / sorted forms: tiled slabs at 32, 36, 40, 48 positions 110 / 128, 117 / 129,
+# 127 / 129, 158 / 132 (the shared expert on its own stream 117 / 129, 125 / 131, 136 / 130), GGUF rows at 32, 34, 36
+# 153 / 168, 161 / 160, 168 / 168 (160 / 168, 166 / 163, 175 / 172).  Half the pairs on 8 experts: tiled 40 122 / 124,
+# rows 33 153 / 154.  Where more tokens share experts the sorted forms are ahead earlier (popularity
+# e^(1.5 N(0,1)): tiled 24 87 / 97, 28 100 / 99, 40 133 / 107).
 MOE_CKPT_PAIR_WALK_MAX_P = {LAYOUT_TILED: 40, LAYOUT_RAW: 32}
 
 
@@ -1083,8 +1087,8 @@ def moe_layer(logits, sg, xs, hres, y, ptbl, ptbl_dn, ptbl_sh, iq4nl, scratch, s
 def moe_layer_ckpt(logits, sg, xs, hres, y, ptbl, ptbl_dn, shared8, gridf, scratch, stream=None, down="q6k",
                    iq4nl=None, pair_walk=None, overlap_shared=None, layout=LAYOUT_RAW):
     """One MoE layer with the reference checkpoint's classes, the same sequence as moe_layer:
-    top-8, then the pair walk (P <= MOE_PAIR_WALK_MAX_P by default) or sort + grouped forms for
-    the IQ3_S gate+up, the down projection -- ``down`` "q6k" (Q6_K slabs, the checkpoint's layers
+    top-8, then the pair walk (by default up to MOE_CKPT_PAIR_WALK_MAX_P[layout] positions, with an
+    IQ4_XS down MOE_PAIR_WALK_MAX_P) or sort + grouped forms for the IQ3_S gate+up, the down projection -- ``down`` "q6k" (Q6_K slabs, the checkpoint's layers
     34/38/39) or "iq4" (IQ4_XS GGUF-row slabs, iq4nl given) -- the Q8_0 shared expert
     (shared8 = (wg, wu, wd) rows), and the combine into y.  overlap_shared as moe_layer's: by
     default the shared expert rides in the routed launches (the pair walk's moe_up3s_pairs_sh /
