@@ -435,7 +435,10 @@ int tlx_moe_combine(const uint16_t* parts, const float* gates, const float* sg, 
  * reference's decode forms accumulate in fp32 FMA-free, its prefill forms in fp16 MMA).  Slabs as
  * the reference's: IQ3_S gate/up slab = 512 gate rows, then 512 up rows from byte 450,560, 880 B a
  * row (k = 2048); Q6_K down slab = 2048 rows of 420 B (raw 210-B blocks, k = 512); slab addresses
- * 2-B aligned.  gridf: the IQ3_S grid as float[512][4], passed at run time as by the reference.
+ * 2-B aligned.  gridf: the IQ3_S grid as float[512][4], passed at run time as by the reference.  The
+ * GEMMs take its levels as fp16 and multiply them by the sub-block scale's 1 + 2 s <= 31 in fp16: exact,
+ * and the operand then fp16 of the fp32 value, for levels of at most 6 significant bits (the format's
+ * are the odd integers up to 15); with other levels the operands round once more.
  * np = number of pairs (8 per position), <= 16384; the sorted forms take tlx_moe_sort's eoff / plist.
  * layout (the routed forms' argument before the stream): TLX_LAYOUT_RAW for slabs of GGUF rows as
  * above, TLX_LAYOUT_TILED for slabs repacked by tlx_pack_iq3s_tiled / tlx_pack_q6k_tiled (same
@@ -467,8 +470,7 @@ int tlx_moe_up3s(const uint64_t* ptbl, const int* eoff, const uint16_t* plist, c
                  const float* gridf, float* ys, int np, int layout, void* stream);
 /* Pair-walk form (no sort): pair p runs expert eids[p].  Replaces gx8e256up
  * (engine/mm/MM_P1_gx8e256up.cu:15-20): gx8e256up(ptbl, eids, xs, gridf, ys).  The decode form:
- * weights go straight to registers, the grid's levels are read as fp16 (exact for the IQ3_S
- * grid's integers); the operands are tlx_moe_up3s's, summed in another k order (within 1e-5). */
+ * weights go straight to registers; the operands are tlx_moe_up3s's, summed in another k order (within 1e-5). */
 int tlx_moe_up3s_pairs(const uint64_t* ptbl, const uint16_t* eids, const float* xs, const float* gridf,
                        float* ys, int np, int layout, void* stream);
 /* Q6_K grouped down over the sorted pairs: parts[pair][2048] = fp16(Wd_e . act[pair]).  Replaces

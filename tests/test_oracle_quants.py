@@ -297,3 +297,21 @@ def test_q80_known_answer_every_int8():
     w = quants.dequant_q8_0(raw, 256)[0]
     want = np.concatenate([q[32 * k:32 * (k + 1)].astype(np.float64) * 2.0 ** -k for k in range(8)])
     assert np.array_equal(w.astype(np.float64), want)
+
+
+def test_iq3s_operand_is_one_rounding():
+    """IQ3_S operands by fp16 multiplies, ((1 + 2 s) * level) * d, are fp16 of the GGUF value d * (1 + 2 s) * level
+    for every sub-block scale s and the grid's levels, the odd integers up to 15: the first product is exact
+    for every level of at most 6 significant bits, and no longer for all of 7."""
+    d = np.arange(0x0400, 0x7C00, dtype=np.uint16).view(np.float16)   # every normal scale
+    mult = 1 + 2 * np.arange(16)
+    exact = [np.array_equal((mult.astype(np.float16) * np.float16(v)).astype(np.int64), mult * v) for v in range(128)]
+    assert all(exact[:64]) and not all(exact[64:])
+    levels = np.unique(synth.iq3s_grid(np.random.default_rng(3)))
+    assert set(levels) <= {1.0 + 2.0 * i for i in range(8)}
+    with np.errstate(over="ignore"):
+        for m in mult:
+            for v in levels:
+                want = (d.astype(np.float64) * float(m) * float(v)).astype(np.float16)
+                got = (np.float16(m) * np.float16(v)) * d
+                assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), (m, v)

@@ -213,7 +213,8 @@ __device__ __forceinline__ void gv_lut_fill(GvLut& L, const float* gridf, int t)
 }
 
 // The 16 weights as fp16 operands, bit for bit the fp16 of gx_decode's values.  IQ3_S and Q8_0: packed
-// fp16 multiplies -- (1 + 2 nib) * level <= 465 and an int8 are exact fp16 integers and d is fp16 itself,
+// fp16 multiplies -- (1 + 2 nib) * level <= 465 (any level of at most 6 significant bits: tlx.h's condition on
+// the grid) and an int8 are exact in fp16 and d is fp16 itself,
 // so the product with d is rounded once, to the reference's operand.  Q6_K: sc * (q - 32) is not exact in
 // fp16; d * sc * (q - 32) has <= 23 bits, exact in f32 (tlx_mix2_f16).  The multiplies are the cheaper:
 // 2.2 ns a wave instruction and SIMD, for two weights, against 6.7 for tlx_mix2_f16's three.
