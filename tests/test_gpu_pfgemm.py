@@ -173,6 +173,9 @@ def _parts_written(ws, mark):
     (256, 5120, 17408, 11, 40),     # 44 slots: 2 each
     (256, 5120, 17408, 8, 0),       # 32 slots: whole tiles
     (512, 256, 4096, 128, 16),      # 2 tiles of 32 chunks, at least 4 chunks a range
+    (512, 256, 512, 128, 8),        # 2 tiles of 4 chunks: 4 ranges of a chunk each
+    (256, 256, 256, 128, 0),        # one tile of 2 chunks: whole
+    (1024, 5120, 2048, 128, 240),   # 80 tiles of 16 chunks: 2 or 3 ranges a tile cost the same
     (2048, 5120, 17408, 128, 384),  # 160 tiles in 256 ranges: two segments a workgroup
     (2048, 5120, 17408, 104, 384),  # the same in the 415 slots that it asks for
     (2048, 5120, 17408, 103, 0),    # one MiB less: whole tiles

@@ -629,10 +629,13 @@ int pf_check(const void* w, const void* x, int M, int N, int K, int layout, int 
 }
 
 // The split tiles' sums: workgroup (st, i, jp) adds the parts of row group i (16 rows per wave row) and
-// column groups jp, jp + 4 of split tile st in range order (fixed: the result does not depend on which
-// range finished first) and applies the epilogue to them.  Bound by the parts' bytes: 16 workgroups a
-// tile, each thread's loads of up to four parts in flight (8 workgroups with one part at a time in
-// flight: M = 256 down 21 us for 21 MB).
+// a pair of column groups of split tile st in range order (fixed: the result does not depend on which
+// range finished first) and applies the epilogue to them.  The pair is a gate group and its up group, else
+// two neighbours: 32 columns, whole 128-B lines of an fp32 output (with groups jp, jp + 4 two workgroups, on
+// different XCDs, wrote each line: K = 2048, N = 8192, M = 1024, two parts a tile, 24.9 us against 20.8).
+// Bound by the parts' bytes: 16 workgroups a tile, each thread's loads of up to four parts in flight.  us,
+// 16 / 8 / 4 workgroups a tile: 20 tiles of 12 parts 12.5 / 11.4 / 15.0, 160 of 2 to 3 32.3 / 30.9 / 33.0, 2 of
+// 8 (FFN) 4.0 / 3.9 / 5.5.
 constexpr int kFixPer = 4 * kMI;
 template <int EPI>
 __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out, const float* __restrict__ res, int N, int nch,
@@ -646,7 +649,9 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out
   const int chunks = sk.r * nch, c0 = st * nch;
   const int g0 = pf_range_of(chunks, sk.G, c0), g1 = pf_range_of(chunks, sk.G, c0 + nch - 1);
   constexpr size_t kSlot = kBM * kBN / 4;
-  const f4_t* part = reinterpret_cast<const f4_t*>(sk.part) + (size_t)(i * 8 + jp) * kThreads + threadIdx.x;
+  // the pair's column groups jg[0], jg[1], in the order of the accumulators
+  const int jg[2] = {kFfn ? jp : 2 * jp, kFfn ? jp + 4 : 2 * jp + 1};
+  const f4_t* part = reinterpret_cast<const f4_t*>(sk.part) + (size_t)(i * 8 + jg[0]) * kThreads + threadIdx.x;
   f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
   const auto add = [&](auto count, int g) {   // parts g .. g + count - 1, all requested first
     constexpr int C = decltype(count)::value;
@@ -655,7 +660,7 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out
     for (int q = 0; q < C; ++q) {
       const f4_t* p = part + (size_t)sk.slot(g + q, st) * kSlot;
       v[q][0] = p[0];
-      v[q][1] = p[4 * kThreads];
+      v[q][1] = p[(kFfn ? 4 : 1) * kThreads];
     }
 #pragma unroll
     for (int q = 0; q < C; ++q) {
@@ -680,7 +685,7 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out
     } else {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const size_t o = (size_t)m * N + nt * kBN + 16 * (8 * wn + jp + 4 * j) + col;
+        const size_t o = (size_t)m * N + nt * kBN + 16 * (8 * wn + jg[j]) + col;
         if constexpr (EPI == PF_RES)
           reinterpret_cast<float*>(out)[o] = res[o] + acc[j][e];
         else
@@ -696,15 +701,17 @@ __global__ __launch_bounds__(kThreads) void pf_fix_kernel(void* __restrict__ out
 // one more round of whole tiles.  Cost in 1/40 chunk (0.1 us; a 128-k chunk of a tile takes about 4 us a
 // CU): the longest range's chunks, 1.5 chunks a segment for its prologue, 1 a part (256 KB written and
 // read again).  Measured, the FFN block (G by equal splits of 2 to 4 a tile -> by this rule): M = 256
-// 284 -> 188 us (down: 80 workgroups -> 240).  With G always one a CU M = 1536 took 873 us against 862.
+// 284 -> 188 us (down: 80 workgroups -> 240).  With G always one a CU M = 1536 took 873 us against 862.  A range
+// has at least 4 chunks, but at most 4 a tile may be shorter (K = 512, one tile: 4 ranges of a chunk 13.6 us,
+// whole 21.4); of equal costs the larger G (K = 2048, N = 5120, M = 1024: 240 ranges 51.4 us, 160 56.8).
 int pf_ranges(int r, int nch, int G0, int64_t slots) {
   const int64_t chunks = (int64_t)r * nch;
   int best = 0;
   int64_t least = 40LL * nch;
   const auto take = [&](int64_t G, int64_t segs, int64_t parts) {
-    if (G <= r || 4 * G > chunks || pf_slots(r, G) > slots) return;
+    if (G <= r || G > chunks || (4 * G > chunks && G > 4 * (int64_t)r) || pf_slots(r, G) > slots) return;
     const int64_t cost = 40 * ((chunks + G - 1) / G) + 60 * segs + parts;
-    if (cost < least) { least = cost; best = (int)G; }
+    if (cost < least || (cost == least && best > 0)) { least = cost; best = (int)G; }
   };
   for (int64_t G = 2 * (int64_t)r; G <= G0; G += r) take(G, 1, G);
   take(G0, 2, r + G0 - 1);
