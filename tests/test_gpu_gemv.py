@@ -361,7 +361,9 @@ def test_attention_variants(gpu, name, M):
     # a launch a matrix, where q's rows fit the LDS with more activation rows than the three together do
     # (K = 4096: 16 against 15; 8192: 8 against 7)
     (4096, 70, 40, 33, 16, True, True), (4096, 70, 40, 33, 16, False, False),
-    (8192, 40, 24, 50, 8, False, False), (8192, 40, 24, 50, 9, True, False)])
+    (8192, 40, 24, 50, 8, False, False), (8192, 40, 24, 50, 9, True, False),
+    # two row groups and more IQ3_XXS bytes than are worth reading twice
+    (5120, 33, 2800, 2803, 13, False, False)])
 def test_qkv_three_formats_one_launch(gpu, K, Nq, Nk, Nv, M, v4, raw):
     from thunderllamax_amd._lib import V_Q4K
     print(f"[case] q6/iq3/q4 K={K} rows {Nq} {Nk} {Nv} M={M} v4={v4} raw={raw}", flush=True)

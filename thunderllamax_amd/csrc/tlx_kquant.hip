@@ -757,6 +757,12 @@ int tlx_kq_mix(int fmt, const void* const* w, uint16_t* const* out, const int* n
   int mc = M;
   while (mc > 1 && k_mix_lds_bytes(fmt, mc, K, v4) > (size_t)kLdsMax) --mc;
   *done = k_mix_lds_bytes(fmt, mc, K, v4) <= (size_t)kLdsMax && mc == k_rows_per_pass(fmt, M, K);
+  // An IQ3_XXS k and v read in a launch of their own are read once for all M rows, here once a row group: worth
+  // it for 8 MB (K = 5120, M = 13, 12288 + 2048 + 2048 rows: 37.0 us apart, 31.6 together), not for 16 (12288 +
+  // 4096 + 4096: 40.1, 42.9).  With a Q4_K v, whose own launches go by row groups too, it always is (12288 +
+  // 16384 + 16384: 75 us apart, 71 together).
+  const int64_t again = (int64_t)((M + mc - 1) / mc - 1) * (n[1] + n[2]) * 98 * (K >> 8);
+  if (!v4 && again > (int64_t)10 << 20) *done = false;
   if (!*done) return TLX_OK;
   KMixArgs a{};
   for (int i = 0; i < 3; ++i) a.seg[i] = KMixSeg{(const uint8_t*)w[i], out[i], n[i], 0, 0};
