@@ -347,7 +347,7 @@ int tlx_moe_topk(const float* logits, uint16_t* eids, float* gates, int P, void*
 int tlx_moe_route(const float* wrt, const float* wsh, const float* h, uint16_t* eids, float* gates,
                   float* sg, int P, void* stream);
 /* The same with the logits through caller-owned memory, f32[P][256], 16-B aligned (written): every
- * router row on a workgroup of its own, then tlx_moe_topk.  The faster form up to about 80 positions;
+ * router row on a workgroup of its own, then tlx_moe_topk.  The faster form up to about 88 positions;
  * the same results bit for bit. */
 int tlx_moe_route_logits(const float* wrt, const float* wsh, const float* h, float* logits, uint16_t* eids,
                          float* gates, float* sg, int P, void* stream);

@@ -141,10 +141,10 @@ def test_moe_route(gpu):
     np.testing.assert_allclose(sg.cpu().numpy(), ref_sg, rtol=1e-5)
 
 
-@pytest.mark.parametrize("P", [1, 3, 4, 5, 80, 81, 96, 97, 257, 1027])
+@pytest.mark.parametrize("P", [1, 3, 4, 5, 40, 41, 88, 89, 96, 97, 257, 1027])
 def test_moe_route_batches(gpu, P):
-    """A workgroup per router row (up to 80 positions; fewer than, as many as and more than its four
-    waves), and every positions-a-workgroup form (1, 4, 8) with a ragged last workgroup: logits in float64 decide
+    """A workgroup per router row (up to 88 positions; fewer than, as many as and more than its four
+    waves, eight waves above 40), and every positions-a-workgroup form (1, 4, 8) with a ragged last workgroup: logits in float64 decide
     the ids where the 8th and 9th are apart by more than fp32 sums of 2048 terms can move (1e-4)."""
     print(f"[case] moe route P={P}", flush=True)
     rng = np.random.default_rng(1200 + P)
@@ -205,7 +205,7 @@ def test_moe_topk_extremes(gpu):
     torch.testing.assert_close(gates[0, :3].cpu(), torch.softmax(torch.tensor([3.0, 2.0, 1.0]), 0), rtol=2e-6, atol=0)
 
 
-@pytest.mark.parametrize("P", [1, 5, 80, 96])
+@pytest.mark.parametrize("P", [1, 5, 41, 88, 96])
 def test_moe_route_forms_agree(gpu, P):
     """The router's results are the same bits on every route: the current stream (given or not), another
     stream, a caller's logits buffer, stream capture (the replays, eager work between them) and the C call.

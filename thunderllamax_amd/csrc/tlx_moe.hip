@@ -50,8 +50,7 @@ __device__ __forceinline__ float wave_max(float v) {   // (fmaxf: NaN only if ev
 }
 // The order of a router row's sum (fp32 products and sums), the same in both kernels below, so that a
 // logit's bits depend on neither: 64 chains of 8 steps a component -- chain (j, piece), j < 16, piece < 4,
-// takes the row's 16-B pieces 32 j + 4 i + piece, i = 0 .. 7 -- then chains j in fours, the four sums of
-// those, and last the pieces.
+// takes the row's 16-B pieces 32 j + 4 i + piece, i = 0 .. 7 -- then a binary tree over j, and last the pieces.
 constexpr int kRtChain = 8;
 __device__ __forceinline__ void rt_step(float4& acc, float4 w, float4 x, bool first) {
   acc.x = first ? w.x * x.x : __builtin_fmaf(w.x, x.x, acc.x);
@@ -71,16 +70,16 @@ __device__ __forceinline__ float rt_row(const float4 (&w)[kRtChain], const float
   float4 acc;
 #pragma unroll
   for (int i = 0; i < kRtChain; ++i) rt_step(acc, w[i], x[i], i == 0);
-  const float q = rt_fold(acc);
-  float g = q + dpp_f<0x104, 0xF>(q);   // row_shl: lane l takes lane l + 4, + 8, + 12 of its 16-lane row
-  g += dpp_f<0x108, 0xF>(q);
-  g += dpp_f<0x10C, 0xF>(q);
-  const uint32_t gb = __builtin_bit_cast(uint32_t, g);
-  const auto r = __builtin_amdgcn_permlane16_swap(gb, gb, false, false);   // row 0: rows 0 and 1; row 2: rows 2 and 3
+  float q = rt_fold(acc);
+  q += dpp_f<0x104, 0xF>(q);   // row_shl: lane l takes lane l + 4, then l + 8, of its 16-lane row
+  q += dpp_f<0x108, 0xF>(q);
+  uint32_t b = __builtin_bit_cast(uint32_t, q);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);   // row 0: rows 0 and 1; row 2: rows 2 and 3
   const uint32_t r0 = r[0], r1 = r[1];   // (values of their own: __builtin_bit_cast of a vector's element takes element 0)
-  const uint32_t r2 = __builtin_amdgcn_permlane32_swap(r0, r0, false, false)[1];   // row 0: row 2's
-  const uint32_t r3 = __builtin_amdgcn_permlane32_swap(r1, r1, false, false)[1];
-  const float v = ((__builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1)) + __builtin_bit_cast(float, r2)) + __builtin_bit_cast(float, r3);
+  float v = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+  b = __builtin_bit_cast(uint32_t, v);
+  const uint32_t r2 = __builtin_amdgcn_permlane32_swap(b, b, false, false)[1];   // row 0: row 2's
+  v += __builtin_bit_cast(float, r2);
   return rt_pieces(v);
 }
 // 16-B piece k4 of wsh, which is 8-B aligned
@@ -141,8 +140,8 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
 // takes NP positions: their h in LDS, wave w the 16 experts 16 w .. , four lanes a row so that a
 // wave's 16-B loads read 64 contiguous bytes a quad (a row per lane, as before, took a quarter of
 // that rate), 16 or 8 loads ahead; every weight feeds NP positions.  The bound at few positions is the
-// 2 MB of wrt through one CU's load path (64 B a clock), at many the reads of h from LDS (16 B a wave and
-// step for 4 FMAs).
+// 2 MB of wrt through one CU's load path (64 B a clock), at many the issue of the FMAs and of the LDS reads of
+// h between them (P = 2048: 92% of the SIMDs' cycles issue, 71% VALU; LDS 59% active).
 constexpr int kRtThreads = 1024, kRtWaves = kRtThreads / TLX_WAVE;
 template <int NP>
 __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
@@ -163,9 +162,7 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __re
     hs[p][k4] = reinterpret_cast<const float4*>(h + (size_t)min(p0 + p, P - 1) * kHid)[k4];   // past P: unused
   }
   __syncthreads();
-  float four[NP], tot[NP];   // the sums of the chains of the present four, and of the fours before
-#pragma unroll
-  for (int p = 0; p < NP; ++p) four[p] = tot[p] = 0.f;
+  float level[4][NP], tot[NP];   // the tree over the chains: a chain, two, four, eight waiting for their like
   // slot u of the ring: step s0 + u's weights, then (once used) step s0 + kRtAhead + u's.  The fences
   // keep each pair of steps' requests behind its uses: without them the scheduler moves the requests
   // to where the loop's end has to wait for all of them.
@@ -180,15 +177,20 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __re
       w[u] = wn[4 * u];
       if (u & 1) __builtin_amdgcn_sched_barrier(0);
       if (u % kRtChain == kRtChain - 1) {
+        const int j = (s0 + u) / kRtChain;
 #pragma unroll
-        for (int p = 0; p < NP; ++p) four[p] += rt_fold(acc[p]);
-      }
-    }
-    if ((s0 + kRtAhead) % (4 * kRtChain) == 0) {
+        for (int p = 0; p < NP; ++p) tot[p] = rt_fold(acc[p]);
+        bool up = true;   // (uniform)
 #pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        tot[p] += four[p];
-        four[p] = 0.f;
+        for (int l = 0; l < 4; ++l) {
+          if (!up) continue;
+          up = (j >> l) & 1;
+#pragma unroll
+          for (int p = 0; p < NP; ++p) {
+            if (up) tot[p] += level[l][p];
+            else level[l][p] = tot[p];
+          }
+        }
       }
     }
   }
@@ -217,19 +219,18 @@ __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __re
 }
 
 // The same logits with a workgroup per router row (row 256 is wsh, whose sums end as sg) and the
-// positions dealt to its four waves: a wave holds the row's 8 KB in 32 registers and reads each
+// positions dealt to its waves: a wave holds the row's 8 KB in 32 registers and reads each
 // position's h against it, two positions in flight.  wrt then comes through every CU's load path
 // instead of one CU's per position; the logits go through memory to moe_topk_kernel.  Both launches, us
-// at P = 1 / 4 / 16 / 64 / 80 / 96: 5.1 / 6.0 / 8.1 / 15.1 / 17.4 / 19.8 against 17.1 / 17.3 / 17.5 / 17.5 / 17.6 /
-// 17.6 of moe_route_kernel (one session, replayed back to back).  Other wave counts, measured at P = 1 / 4 / 16 /
-// 64 / 128 with another order of the sums: 1 wave 5.6 / 6.9 / 12.2 / 31 / 57, 4 waves 5.7 / 6.5 / 8.8 / 15.9 / 24.9,
-// 8 waves 5.5 / 6.4 / 9.2 / 15.3 / 23.5.  Bound by the two launches at few positions, from 16 on by h, which
-// every workgroup reads whole (8 KB a position and CU).  The sum of a position's chains beside the products of
-// the next position's: 14.7 at P = 64, but 6.2 / 8.2 at 4 / 16.
-constexpr int kLgWaves = 4;
-__global__ __launch_bounds__(kLgWaves * TLX_WAVE) void moe_logits_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
-                                                                         const float* __restrict__ h, float* __restrict__ logits,
-                                                                         float* __restrict__ sg, int P) {
+// at P = 4 / 16 / 32 / 40 / 64 / 80 / 88: 4 waves 6.0 / 8.0 / 10.5 / 11.6 / 15.2 / 17.5 / 19.0, 8 waves 5.9 / 8.5 /
+// 10.7 / 11.6 / 14.6 / 16.6 / 17.6, 16 waves 6.0 / 10.2 / 12.3 / 13.2 / 16.2 / 18.3 / 19.2, moe_route_kernel 17.4 .. 17.6
+// (one session, replayed back to back): 4 waves up to kLgWide positions, then 8.  Bound by the two launches at few
+// positions, from 16 on by h, which every workgroup reads whole (8 KB a position and CU).
+constexpr int kLgWide = 40;
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * TLX_WAVE) void moe_logits_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,
+                                                                      const float* __restrict__ h, float* __restrict__ logits,
+                                                                      float* __restrict__ sg, int P) {
   const int row = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int k0 = 32 * (lane >> 2) + (lane & 3);   // (a quad's loads are 64 contiguous bytes)
   const float4* hp = reinterpret_cast<const float4*>(h) + k0;
@@ -240,8 +241,8 @@ __global__ __launch_bounds__(kLgWaves * TLX_WAVE) void moe_logits_kernel(const f
     w[i] = row < kE ? reinterpret_cast<const float4*>(wrt + (size_t)row * kHid)[k0 + 4 * i] : rt_wsh(wsh, k0 + 4 * i);
 #pragma unroll
   for (int i = 0; i < kRtChain; ++i) x[i] = hp[(size_t)wave * (kHid / 4) + 4 * i];
-  for (int p = wave; p < P; p += kLgWaves) {
-    const float4* hn = hp + (size_t)min(p + kLgWaves, P - 1) * (kHid / 4);   // past the end: the last position again
+  for (int p = wave; p < P; p += WAVES) {
+    const float4* hn = hp + (size_t)min(p + WAVES, P - 1) * (kHid / 4);   // past the end: the last position again
     float4 n[kRtChain];
 #pragma unroll
     for (int i = 0; i < kRtChain; ++i) n[i] = hn[4 * i];
@@ -1247,8 +1248,8 @@ extern "C" int tlx_moe_topk(const float* logits, uint16_t* eids, float* gates, i
 }
 
 // Positions a workgroup by batch, the fewest that keep the grid within one workgroup a CU (256):
-// us at 1 / 4 / 8 positions a workgroup: P = 4 17.4 / 21.7 / 42.2, 256 20.7 / 22.3 / 43.3, 300 35.4 /
-// 22.5 / 43.5, 1024 74 / 29.8 / 44.5, 1100 89 / 47.3 / 44.7, 2048 147 / 56.3 / 47.3.  (A row per lane and one
+// us at 1 / 4 / 8 positions a workgroup: P = 4 17.4 / 21.7 / 42, 256 20.7 / 22.3 / 43, 300 35.4 /
+// 22.5 / 43, 1024 74 / 28.3 / 44, 1100 89 / 47 / 39.5, 2048 147 / 56 / 46.1.  (A row per lane and one
 // position a workgroup: 62 us at P = 4, 525 at 2048.)
 constexpr int kRt1 = 256, kRt4 = 1024;
 
@@ -1267,7 +1268,8 @@ extern "C" int tlx_moe_route_logits(const float* wrt, const float* wsh, const fl
   TLX_RET_IF(P < 1, TLX_E_ARG);
   TLX_RET_IF(!tlx_aligned(wrt, 16) || !tlx_aligned(h, 16) || !tlx_aligned(wsh, 8) || !tlx_aligned(logits, 16), TLX_E_ALIGN);
   const hipStream_t st = (hipStream_t)stream;
-  moe_logits_kernel<<<kE + 1, kLgWaves * TLX_WAVE, 0, st>>>(wrt, wsh, h, logits, sg, P);
+  if (P <= kLgWide) moe_logits_kernel<4><<<kE + 1, 4 * TLX_WAVE, 0, st>>>(wrt, wsh, h, logits, sg, P);
+  else moe_logits_kernel<8><<<kE + 1, 8 * TLX_WAVE, 0, st>>>(wrt, wsh, h, logits, sg, P);
   const int rc = tlx_launch_status();
   TLX_RET_IF(rc != TLX_OK, rc);
   return tlx_moe_topk(logits, eids, gates, P, stream);

@@ -632,8 +632,8 @@ def moe_topk(logits, eids, gates, stream=None):
 
 
 # Largest batch the router takes with a workgroup per router row and the logits in memory: device time
-# at 64 / 80 / 96 positions 15.1 / 17.4 / 19.8 us against 17.5 / 17.6 / 17.6 with whole positions a workgroup.
-MOE_ROUTE_LOGITS_MAX_P = 80
+# at 64 / 80 / 88 / 96 positions 14.6 / 16.6 / 17.6 / 19.1 us against 17.5 with whole positions a workgroup.
+MOE_ROUTE_LOGITS_MAX_P = 88
 
 
 def moe_route(wrt, wsh, h, eids, gates, sg, stream=None, logits=None):
