@@ -420,7 +420,8 @@ __global__ __launch_bounds__(kWaves * TLX_WAVE) void kq_gemv16_kernel(const KqAr
 // end together and all are resident at once (kq_mix_plan).  At M = 1 / 4 / 8 / 11 / 16 the three
 // matrices take 15.7 / 16.4 / 17.2 / 18.0 / 33.4 us (26.8 / 28.6 / 32.8 / 33.8 / 55.5 as launches of
 // their own; from M = 13 on two row groups read the weights twice).  57 MB in 15.7 us is 3.6 TB/s:
-// bound by the loads a CU keeps in flight (two items a wave) and the launch's ~4 us start and drain.
+// bound by two waves a SIMD, whose decode (65% of the SIMDs' cycles issue, 40% VALU) and load waits (39% of a
+// wave's cycles) overlap in part, and by the launch's ~4 us start and drain.
 // Held to 128 VGPRs, so that two workgroups fit a CU, it is slower at every M (17.1 .. 35.8 us).
 
 // IQ3_XXS rows (GGUF blocks or packed rows), the arithmetic and the block -> wave split of the

@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
 // wave's 16-B loads read 64 contiguous bytes a quad (a row per lane, as before, took a quarter of
 // that rate), 16 or 8 loads ahead; every weight feeds NP positions.  The bound at few positions is the
 // 2 MB of wrt through one CU's load path (64 B a clock), at many the issue of the FMAs and of the LDS reads of
-// h between them (P = 2048: 92% of the SIMDs' cycles issue, 71% VALU; LDS 59% active).
+// h between them (P = 2048: VALU 85% of the cycles, LDS 64%).
 constexpr int kRtThreads = 1024, kRtWaves = kRtThreads / TLX_WAVE;
 template <int NP>
 __global__ __launch_bounds__(kRtThreads) void moe_route_kernel(const float* __restrict__ wrt, const float* __restrict__ wsh,

@@ -783,7 +783,8 @@ int gv_launch(const GxArgs& a, int items, hipStream_t st) {
 // staged form's 110 / 164 / 166 / 179; all positions on the same 8 experts, 64 / 256 / 512: 34 / 61 / 96
 // against 65 / 158 / 302.  (A workgroup walking all of its expert's tokens, 16 at a time: 57 / 85 / 102 / 148
 // and 93 / 353 / 694: the hottest expert was the launch; 32 tokens a workgroup 55 / 83 / 103 / 148 and 72 /
-// 92 / 134.)  Two units in flight and 128 VGPRs, so that two workgroups fit a CU: with all four units 45 /
+// 92 / 134.)  Bound by the issue of the decode and its table reads: at P = 256 97% of the SIMDs' cycles issue, 79%
+// VALU; LDS 52% active, half of that bank conflicts of the grid lookups.  Two units in flight and 128 VGPRs, so that two workgroups fit a CU: with all four units 45 /
 // 64 / 81 / 111, k over four waves instead of two 69 / 104 / 143 / 208.
 
 // item i of the tokens past every expert's first kGvTok: its expert and first pair, or false past the
